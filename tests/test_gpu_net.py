@@ -262,3 +262,28 @@ def test_training_steps_reduce_the_loss(env):
     assert all(np.isfinite(losses))
     net.release(plan)
     plan.close()
+
+
+@pytest.mark.parametrize("ntiles", [1, 15, 17, 63, 65, 1023, 1025])
+def test_grad_w_partial_counts(env, ntiles):
+    """One image of `ntiles` 4 x 16 tiles gives min(ntiles, 1024) partials: the
+    edges of the grouped sum.  Entries in {-1, 0, 1} make every sum an integer
+    below 2^24, so FP32 is exact in any order."""
+    torch, learned, ctx = env
+    rng = np.random.default_rng(ntiles)
+    R, C = 4, 16 * ntiles
+    plan = learned.Plan(ctx, rows=[R], cols=[C])
+    x = rng.integers(-1, 2, size=(R, C, 32)).astype(np.float64)
+    g = rng.integers(-1, 2, size=(R, C, 32)).astype(np.float64)
+    L = learned._bind(ctx.L)
+    work = torch.zeros(int(L.imau_net_grad_w_work(plan.h, 0, 32, 32)), dtype=torch.float32, device="cuda")
+    dw = torch.zeros(9 * 32 * 32, dtype=torch.float32, device="cuda")
+    db = torch.zeros(32, dtype=torch.float32, device="cuda")
+    g_d, x_d = dev(torch, bits(g).ravel()), dev(torch, bits(x).ravel())
+    ctx._check(L.imau_net_conv_grad_w(ctx.h, plan.h, 0, 32, 32, learned._ptr(g_d), learned._ptr(x_d),
+                                      learned._ptr(dw), learned._ptr(db), learned._ptr(work)))
+    ctx._check(L.imau_net_sync(ctx.h))
+    rw, rb = NO.conv_grad_w(g, x)
+    assert np.array_equal(dw.cpu().numpy().reshape(9, 32, 32), rw)
+    assert np.array_equal(db.cpu().numpy(), rb)
+    plan.close()
