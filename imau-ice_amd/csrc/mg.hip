@@ -436,70 +436,174 @@ __global__ void __launch_bounds__(IMAU_WG) k_cgs(CLevelT<T> L, int color, const 
   }
 }
 
-// One fused Gauss-Seidel sweep of a coarse level: the tile (IMAU_TI x IMAU_TJ)
-// plus a halo of 4 cells is staged in LDS from (xiu, xiv) (zero when xiu is
-// null), the four colour phases update shrinking regions (exact up to 3 - p
-// cells beyond the tile after phase p) and the tile is written to (xou, xov),
-// a different buffer, so the result equals four in-place colour launches.
-#define CH 4
-#define CRI (IMAU_TI + 2 * CH)
-#define CRJ (IMAU_TJ + 2 * CH)
+// Fused sweeps of a coarse level, one launch each way.  A tile (IMAU_TI x
+// IMAU_TJ) plus a halo of H cells is held in LDS; the four colour phases update
+// shrinking regions (after phase p the values are exact up to H - 1 - p cells
+// beyond the tile, because every row couples only neighbours at distance one).
+//   k_cdown: the pre-smoothing sweep from zero (H = 5: exact one cell beyond the
+//     tile), the residual of the tile and its restriction to the next level;
+//   k_cup: the iterate plus the prolonged next level, staged as the sum, and
+//     the reversed sweep (H = 4), written to the second buffer.
+// The results equal one launch per colour, k_crestrict and k_cprolong.
+//
+// Coarse levels are bound by the latency of their loads, not by bytes: a level
+// of a 401 x 41 grid is a handful of workgroups.  So each thread owns at most
+// two rows of a colour (CTH threads cover a colour's region, the first one in
+// two steps), the rows' coefficients are loaded into registers for all four
+// phases at once before the first barrier, and the phases touch only LDS.
+// Neighbours outside the level read the LDS halo, which is zero there, with a
+// zero coefficient (the Galerkin sums put nothing into such slots), so no row
+// tests its neighbours.  Measured on the 401 x 41 channel (FP64, one V-cycle
+// has three such levels): a sweep and a restriction kernel, 13.9 + 20.5 us,
+// became k_cdown, 6.6 us; a prolongation and a sweep kernel, 4.6 + 13.9 us,
+// became k_cup, 6.9 us (12 ice caps of 96-512 cells a side, FP32: 17 + 29 ->
+// 8.1 us down, 4.7 + 17 -> 7.9 us up).
+#define CTH 512
+static_assert((IMAU_TI + 6) * (IMAU_TJ / 2 + 3) <= CTH && (IMAU_TI + 8) * (IMAU_TJ / 2 + 4) <= 2 * CTH,
+              "a colour phase has at most one row per thread, the first of k_cdown two");
 template <class T>
-__global__ void __launch_bounds__(IMAU_WG) k_cgs_fused(CLevelT<T> L, const T *__restrict__ xiu,
-                                                       const T *__restrict__ xiv, T *__restrict__ xou,
-                                                       T *__restrict__ xov, int reverse,
-                                                       const int *__restrict__ active) {
-  __shared__ T sx[2][CRI * CRJ];
+struct CRow {
+  T cf[9], b;
+  int l;     // LDS index of the cell, -1: no row
+  bool in;   // the cell lies in the tile
+};
+
+// row of phase region cell q (region half-width r around the tile, halo H)
+template <class T, int H, int R, int COLOR>
+__device__ __forceinline__ void crow_load(const CLevelT<T> &L, const CMember &cm, const Tile &t, int q, CRow<T> &row) {
+  constexpr int RH = IMAU_TJ / 2 + R, N = (IMAU_TI + 2 * R) * RH, CRJ = IMAU_TJ + 2 * H, COMP = COLOR >> 1;
+  row.l = -1;
+  row.in = false;
+  if (q >= N) return;
+  const int Ib = t.i0 - H, Jb = t.j0 - H;
+  const int li = H - R + q / RH;
+  const int lj = H - R + 2 * (q % RH) + ((COLOR ^ (Ib + li + Jb + H - R)) & 1);
+  const int I = Ib + li, J = Jb + lj;
+  if (!cvalid(cm, COMP, J, I)) return;
+  const long long p = cp2(cm, J, I);
+  const T *cf = COMP == 0 ? L.cu : L.cv;
+#pragma unroll
+  for (int k = 0; k < 9; ++k) row.cf[k] = cf[k * L.na + p];
+  row.b = (COMP == 0 ? L.bu : L.bv)[p];
+  row.l = li * CRJ + lj;
+  row.in = li >= H && li < H + IMAU_TI && lj >= H && lj < H + IMAU_TJ;
+}
+
+// off-diagonal sum of a row from the LDS iterate (su, sv)
+template <class T, int COMP, int CRJ>
+__device__ __forceinline__ T crow_sum(const CRow<T> &row, const T *su, const T *sv) {
+  T S = (T)0.0;
+#pragma unroll
+  for (int k = 1; k < 9; ++k) {
+    int cc, dj, di;
+    slot_pos(COMP, k, 0, 0, cc, dj, di);
+    S += row.cf[k] * (cc == 0 ? su : sv)[row.l + di * CRJ + dj];
+  }
+  return S;
+}
+
+template <class T, int COMP, int CRJ>
+__device__ __forceinline__ void crow_gs(const CRow<T> &row, T *su, T *sv) {
+  if (row.l < 0) return;
+  const T S = crow_sum<T, COMP, CRJ>(row, su, sv);
+  (COMP == 0 ? su : sv)[row.l] = (row.cf[0] != (T)0.0) ? mdiv(row.b - S, row.cf[0]) : (T)0.0;
+}
+
+template <class T>
+__global__ void __launch_bounds__(CTH) k_cdown(CLevelT<T> L, CLevelT<T> N, const int *__restrict__ active) {
+  constexpr int H = 5, CRI = IMAU_TI + 2 * H, CRJ = IMAU_TJ + 2 * H;
+  __shared__ T su[CRI * CRJ], sv[CRI * CRJ], sr[2][IMAU_TI * IMAU_TJ];
   const Tile t = L.tiles[imau_xcd_tile()];
   if (!active[t.g] || L.depth[t.g] <= L.lev) return;
   const CMember cm = L.mem[t.g];
-  const int Ib = t.i0 - CH, Jb = t.j0 - CH;
-  const int tid = threadIdx.y * IMAU_TJ + threadIdx.x;
-  for (int q = tid; q < CRI * CRJ; q += IMAU_WG) {
-    const int li = q / CRJ, lj = q - li * CRJ;
-    const int I = Ib + li, J = Jb + lj;
-    T a = (T)0.0, b = (T)0.0;
-    if (xiu) {
-      if (cvalid(cm, 0, J, I)) a = xiu[cp2(cm, J, I)];
-      if (cvalid(cm, 1, J, I)) b = xiv[cp2(cm, J, I)];
-    }
-    sx[0][q] = a;
-    sx[1][q] = b;
+  const int tid = threadIdx.x;
+  CRow<T> r0, r0b, r1, r2, r3;
+  crow_load<T, H, 4, 0>(L, cm, t, tid, r0);
+  crow_load<T, H, 4, 0>(L, cm, t, tid + CTH, r0b);
+  crow_load<T, H, 3, 1>(L, cm, t, tid, r1);
+  crow_load<T, H, 2, 2>(L, cm, t, tid, r2);
+  crow_load<T, H, 1, 3>(L, cm, t, tid, r3);
+  for (int q = tid; q < CRI * CRJ; q += CTH) {
+    su[q] = (T)0.0;
+    sv[q] = (T)0.0;
+  }
+  for (int q = tid; q < IMAU_TI * IMAU_TJ; q += CTH) {
+    sr[0][q] = (T)0.0;
+    sr[1][q] = (T)0.0;
   }
   __syncthreads();
-  for (int ph = 0; ph < 4; ++ph) {
-    const int color = reverse ? 3 - ph : ph;
-    const int comp = color >> 1;
-    const int r = CH - 1 - ph;
-    // lanes take the RW / 2 cells of this colour in each row of the region
-    // (same-component couplings are 5-point, so cells of one colour do not couple)
-    const int RW = IMAU_TJ + 2 * r, RH = RW / 2, n = (IMAU_TI + 2 * r) * RH;
-    const T *cf = comp == 0 ? L.cu : L.cv;
-    for (int q = tid; q < n; q += IMAU_WG) {
-      const int li = CH - r + q / RH;
-      const int lj = CH - r + 2 * (q % RH) + ((color ^ (Ib + li + Jb + CH - r)) & 1);
-      const int I = Ib + li, J = Jb + lj;
-      if (!cvalid(cm, comp, J, I)) continue;
-      const long long p = cp2(cm, J, I);
-      const T D = cf[p];
-      T S = (T)0.0;
-#pragma unroll
-      for (int k = 1; k < 9; ++k) {
-        int cc, JJ, II;
-        slot_pos(comp, k, J, I, cc, JJ, II);
-        if (!cvalid(cm, cc, JJ, II)) continue;
-        S += cf[k * L.na + p] * sx[cc][(II - Ib) * CRJ + (JJ - Jb)];
-      }
-      const T bb = (comp == 0 ? L.bu : L.bv)[p];
-      sx[comp][li * CRJ + lj] = (D != (T)0.0) ? mdiv(bb - S, D) : (T)0.0;
-    }
-    __syncthreads();
+  crow_gs<T, 0, CRJ>(r0, su, sv);
+  crow_gs<T, 0, CRJ>(r0b, su, sv);
+  __syncthreads();
+  crow_gs<T, 0, CRJ>(r1, su, sv);
+  __syncthreads();
+  crow_gs<T, 1, CRJ>(r2, su, sv);
+  __syncthreads();
+  crow_gs<T, 1, CRJ>(r3, su, sv);
+  __syncthreads();
+  // residual of the tile's rows
+  auto res = [&](const CRow<T> &row, T S, const T *x, T *out) {
+    const int li = row.l / CRJ - H, lj = row.l % CRJ - H;
+    out[li * IMAU_TJ + lj] = row.b - S - row.cf[0] * x[row.l];
+  };
+  if (r0.in) res(r0, crow_sum<T, 0, CRJ>(r0, su, sv), su, sr[0]);
+  if (r0b.in) res(r0b, crow_sum<T, 0, CRJ>(r0b, su, sv), su, sr[0]);
+  if (r1.in) res(r1, crow_sum<T, 0, CRJ>(r1, su, sv), su, sr[0]);
+  if (r2.in) res(r2, crow_sum<T, 1, CRJ>(r2, su, sv), sv, sr[1]);
+  if (r3.in) res(r3, crow_sum<T, 1, CRJ>(r3, su, sv), sv, sr[1]);
+  for (int q = tid; q < IMAU_TI * IMAU_TJ; q += CTH) {
+    const int li = q / IMAU_TJ, lj = q % IMAU_TJ, I = t.i0 + li, J = t.j0 + lj;
+    if (cvalid(cm, 0, J, I)) L.xu[cp2(cm, J, I)] = su[(li + H) * CRJ + lj + H];
+    if (cvalid(cm, 1, J, I)) L.xv[cp2(cm, J, I)] = sv[(li + H) * CRJ + lj + H];
   }
-  for (int q = tid; q < IMAU_TI * IMAU_TJ; q += IMAU_WG) {
-    const int li = CH + q / IMAU_TJ, lj = CH + q % IMAU_TJ;
-    const int I = Ib + li, J = Jb + lj;
-    if (cvalid(cm, 0, J, I)) xou[cp2(cm, J, I)] = sx[0][li * CRJ + lj];
-    if (cvalid(cm, 1, J, I)) xov[cp2(cm, J, I)] = sx[1][li * CRJ + lj];
+  __syncthreads();
+  const CMember nm = N.mem[t.g];
+  for (int q = tid; q < 2 * (IMAU_TI / 2) * (IMAU_TJ / 2); q += CTH) {
+    const int comp = q / ((IMAU_TI / 2) * (IMAU_TJ / 2)), c = q % ((IMAU_TI / 2) * (IMAU_TJ / 2));
+    const int li = c / (IMAU_TJ / 2), lj = c % (IMAU_TJ / 2), I = t.i0 / 2 + li, J = t.j0 / 2 + lj;
+    if (!cvalid(nm, comp, J, I)) continue;
+    const T *s = sr[comp] + 2 * li * IMAU_TJ + 2 * lj;
+    (comp == 0 ? N.bu : N.bv)[cp2(nm, J, I)] = (((s[0] + s[IMAU_TJ]) + s[1]) + s[IMAU_TJ + 1]);
+  }
+}
+
+// L.xu / L.xv: the pre-smoothed iterate; N.xu / N.xv: the next level's result;
+// the post-smoothed iterate goes to (xou, xov)
+template <class T>
+__global__ void __launch_bounds__(CTH) k_cup(CLevelT<T> L, CLevelT<T> N, T *__restrict__ xou, T *__restrict__ xov,
+                                            const int *__restrict__ active) {
+  constexpr int H = 4, CRI = IMAU_TI + 2 * H, CRJ = IMAU_TJ + 2 * H;
+  __shared__ T su[CRI * CRJ], sv[CRI * CRJ];
+  const Tile t = L.tiles[imau_xcd_tile()];
+  if (!active[t.g] || L.depth[t.g] <= L.lev) return;
+  const CMember cm = L.mem[t.g], nm = N.mem[t.g];
+  const int tid = threadIdx.x;
+  CRow<T> r0, r1, r2, r3;
+  crow_load<T, H, 3, 3>(L, cm, t, tid, r0);
+  crow_load<T, H, 2, 2>(L, cm, t, tid, r1);
+  crow_load<T, H, 1, 1>(L, cm, t, tid, r2);
+  crow_load<T, H, 0, 0>(L, cm, t, tid, r3);
+  for (int q = tid; q < CRI * CRJ; q += CTH) {
+    const int I = t.i0 - H + q / CRJ, J = t.j0 - H + q % CRJ;
+    T a = (T)0.0, b = (T)0.0;
+    if (cvalid(cm, 0, J, I)) a = L.xu[cp2(cm, J, I)] + N.xu[cp2(nm, J >> 1, I >> 1)];
+    if (cvalid(cm, 1, J, I)) b = L.xv[cp2(cm, J, I)] + N.xv[cp2(nm, J >> 1, I >> 1)];
+    su[q] = a;
+    sv[q] = b;
+  }
+  __syncthreads();
+  crow_gs<T, 1, CRJ>(r0, su, sv);
+  __syncthreads();
+  crow_gs<T, 1, CRJ>(r1, su, sv);
+  __syncthreads();
+  crow_gs<T, 0, CRJ>(r2, su, sv);
+  __syncthreads();
+  crow_gs<T, 0, CRJ>(r3, su, sv);
+  __syncthreads();
+  for (int q = tid; q < IMAU_TI * IMAU_TJ; q += CTH) {
+    const int li = q / IMAU_TJ, lj = q % IMAU_TJ, I = t.i0 + li, J = t.j0 + lj;
+    if (cvalid(cm, 0, J, I)) xou[cp2(cm, J, I)] = su[(li + H) * CRJ + lj + H];
+    if (cvalid(cm, 1, J, I)) xov[cp2(cm, J, I)] = sv[(li + H) * CRJ + lj + H];
   }
 }
 
@@ -985,16 +1089,12 @@ void coarse_fused_t(hipStream_t s, const imau::MGPlan &P, const int *act) {
     if (P.levels[l].ends)
       hipLaunchKernelGGL(k_coarsest<T>, dim3(P.ngrids), dim3(1024), 0, s, C2, act, P.coarsest_sweeps);
     if (l + 1 == nl) break;
-    hipLaunchKernelGGL(k_cgs_fused<T>, dim3(C.ntiles), wg(), 0, s, C, (const T *)nullptr, (const T *)nullptr, C.xu,
-                       C.xv, 0, act);
-    const CLevelT<T> N = view<T>(P, l + 1);
-    hipLaunchKernelGGL(k_crestrict<T>, dim3(N.ntiles), wg(), 0, s, C, N, act);
+    hipLaunchKernelGGL(k_cdown<T>, dim3(C.ntiles), dim3(CTH), 0, s, C, view<T>(P, l + 1), act);
   }
   for (int l = nl - 2; l >= 0; --l) {
-    const CLevelT<T> C = view<T>(P, l), N2 = view2<T>(P, l + 1);
-    hipLaunchKernelGGL(k_cprolong<T>, dim3(C.ntiles), wg(), 0, s, C, N2, act);
-    hipLaunchKernelGGL(k_cgs_fused<T>, dim3(C.ntiles), wg(), 0, s, C, (const T *)C.xu, (const T *)C.xv,
-                       C.bv + C.na, C.bv + 2 * C.na, 1, act);
+    const CLevelT<T> C = view<T>(P, l);
+    hipLaunchKernelGGL(k_cup<T>, dim3(C.ntiles), dim3(CTH), 0, s, C, view2<T>(P, l + 1), C.bv + C.na,
+                       C.bv + 2 * C.na, act);
   }
 }
 
