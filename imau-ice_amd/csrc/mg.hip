@@ -175,51 +175,73 @@ __device__ __forceinline__ bool fine_valid(const Member &m, int comp, int j, int
 // Galerkin products
 // ---------------------------------------------------------------------------
 // fine (level 0, FP64 coefficients) -> level 1
-// One level-1 cell, the components not marked plain: every coupling's
-// unknown is mapped to its aggregate (fine_agg) and slot at run time.
-template <class T, int CROSS>
-__device__ __forceinline__ void gal0_cell(const Member &m, const KP &kp, const CoefT<double> &c, const CLevelT<T> &L,
-                                          const CMember &cm, int J, int I, long long pc, int fl) {
-  for (int comp = 0; comp < 2; ++comp) {
-    if (!cvalid(cm, comp, J, I) || ((fl >> comp) & 1)) continue;
-    double cf[9] = {0, 0, 0, 0, 0, 0, 0, 0, 0};
-    for (int dj = 0; dj < 2; ++dj)
-      for (int di = 0; di < 2; ++di) {
-        const int j = 2 * J + dj, i = 2 * I + di;
-        if (!fine_valid(m, comp, j, i)) continue;
-        const uint8_t rt = comp == 0 ? c.rt_u[p2(m, j, i)] : c.rt_v[p2(m, j, i)];
-        if (!in_row(rt)) continue;
-        auto acc = [&](int cc, int oj, int oi, double val) {
-          int Jc, Ic;
-          if (!fine_agg(m, c.rt_u, c.rt_v, cc, j + oj, i + oi, Jc, Ic)) return;
-          const int s = agg_slot(comp, cc, Jc - J, Ic - I);
-          if (s >= 0) cf[s] += val;
-        };
-        if (comp == 0) u_couplings<CROSS>(m, kp, c, j, i, rt, acc);
-        else v_couplings<CROSS>(m, kp, c, j, i, rt, acc);
-      }
-    T *dst = comp == 0 ? L.cu : L.cv;
-#pragma unroll
-    for (int k = 0; k < 9; ++k) dst[k * L.na + pc] = (T)cf[k];
-  }
-}
-
 // fine -> level 1 on the cells that are not plain (boundary rows, calving
 // fronts, zero rows and their neighbours): a compact list built with the
-// flags, so no wavefront of the interior waits for one such lane
+// flags, so no wavefront of the interior waits for one such lane.
+// Every coupling's unknown is mapped to its aggregate (fine_agg) and slot at
+// run time, a chain of three dependent loads (row type, the unknown's row type,
+// for 'infinite' boundaries its source's).  Bound by that latency: one thread
+// per cell walked its eight rows and their couplings in turn (34-48 us, whatever
+// the size); here eight lanes share a cell (component x fine row), a row's
+// couplings are gathered first so that their loads are in flight together, and
+// the four rows' sums are added across lanes in the rows' order: 10.7 us on the
+// 401 x 41 channel (36 before), 14.6 us on 12 caps of 96-512 cells (46 before).
 template <class T, int CROSS>
 __global__ void __launch_bounds__(256) k_gal0_list(const Member *__restrict__ mem, const KP kp, const CoefT<double> c,
                                                    CLevelT<T> L, const int *__restrict__ active,
                                                    const uint8_t *__restrict__ plain, const int2 *__restrict__ list,
                                                    int n) {
-  const int q = (int)(blockIdx.x * 256 + threadIdx.x);
-  if (q >= n) return;
-  const int2 e = list[q];
-  if (!active[e.x]) return;
+  const int idx = (int)(blockIdx.x * 256 + threadIdx.x);
+  const int comp = (idx >> 2) & 1, dj = (idx >> 1) & 1, di = idx & 1;
+  const int2 e = list[min(idx >> 3, n - 1)];
   const CMember cm = L.mem[e.x];
+  const Member m = mem[e.x];
   const int I = e.y / cm.ny, J = e.y - I * cm.ny;
   const long long pc = cm.off + e.y;
-  gal0_cell<T, CROSS>(mem[e.x], kp, c, L, cm, J, I, pc, plain[pc]);
+  const bool own = (idx >> 3) < n && active[e.x] && cvalid(cm, comp, J, I) && !((plain[pc] >> comp) & 1);
+  double cf[9] = {0, 0, 0, 0, 0, 0, 0, 0, 0};
+  const int j = 2 * J + dj, i = 2 * I + di;
+  if (own && fine_valid(m, comp, j, i)) {
+    const uint8_t rt = comp == 0 ? c.rt_u[p2(m, j, i)] : c.rt_v[p2(m, j, i)];
+    if (in_row(rt)) {
+      int cc[9], jj[9], ii[9], num = 0;
+      double val[9];
+#pragma unroll
+      for (int k = 0; k < 9; ++k) { cc[k] = comp; jj[k] = j; ii[k] = i; val[k] = 0.0; }
+      auto put = [&](int c2, int oj, int oi, double v) {
+        cc[num] = c2; jj[num] = j + oj; ii[num] = i + oi; val[num] = v;
+        ++num;
+      };
+      if (comp == 0) u_couplings<CROSS>(m, kp, c, j, i, rt, put);
+      else v_couplings<CROSS>(m, kp, c, j, i, rt, put);
+      uint8_t rk[9];
+#pragma unroll
+      for (int k = 0; k < 9; ++k) rk[k] = (cc[k] == 0 ? c.rt_u : c.rt_v)[p2(m, jj[k], ii[k])];
+#pragma unroll
+      for (int k = 0; k < 9; ++k) {
+        if (rk[k] == RT_BND_INF) {
+          int jo, io;
+          bnd_src(rk[k], ii[k], jj[k], cc[k] == 0 ? m.nx - 2 : m.nx - 1, cc[k] == 0 ? m.ny - 1 : m.ny - 2, jo, io);
+          jj[k] = jo;
+          ii[k] = io;
+          rk[k] = (cc[k] == 0 ? c.rt_u : c.rt_v)[p2(m, jo, io)];
+        }
+        const int s = in_row(rk[k]) ? agg_slot(comp, cc[k], (jj[k] >> 1) - J, (ii[k] >> 1) - I) : -1;
+#pragma unroll
+        for (int q = 0; q < 9; ++q) cf[q] += (q == s) ? val[k] : 0.0;
+      }
+    }
+  }
+  T *dst = comp == 0 ? L.cu : L.cv;
+#pragma unroll
+  for (int k = 0; k < 9; ++k) {
+    // the rows' order (dj, di) = (0,0), (0,1), (1,0), (1,1)
+    double s = __shfl(cf[k], 0, 4);
+    s += __shfl(cf[k], 1, 4);
+    s += __shfl(cf[k], 2, 4);
+    s += __shfl(cf[k], 3, 4);
+    if (own && (idx & 3) == 0) dst[k * L.na + pc] = (T)s;
+  }
 }
 
 // Plain aggregates: all four fine rows of a level-1 aggregate of component
@@ -293,7 +315,7 @@ __device__ __forceinline__ void gal_plain_row(const Member &m, const KP &kp, con
 }
 
 // fine -> level 1 on the plain aggregates: the same sums in the same order as
-// k_gal0, with straight-line loads and no aggregate look-ups
+// k_gal0_list, with straight-line loads and no aggregate look-ups
 template <class T, int CROSS, int COMP>
 __device__ __forceinline__ void gal_plain(const Member &m, const KP &kp, const CoefT<double> &c, const CLevelT<T> &L,
                                           int J, int I, long long pc) {
@@ -324,25 +346,46 @@ __global__ void __launch_bounds__(IMAU_WG) k_gal0_plain(const Member *__restrict
   }
 }
 
-// one fine cell (2J+DJ, 2I+DI) of a coarse cell whose fine cells and
-// couplings all lie inside the level: slot and target are constants
-template <class T, int COMP, int DJ, int DI>
-__device__ __forceinline__ void galc_plain(const CLevelT<T> &Fl, const CMember &fm, int J, int I, double (&cf)[9]) {
-  const long long pf = cp2(fm, 2 * J + DJ, 2 * I + DI);
+// level l (Fl) -> level l+1 (L), accumulated in FP64; blockIdx.y is the
+// component.  Slot k of a fine row addresses the unknown at constant offsets,
+// so its coarse slot is a constant, at the level's edges too: a slot whose
+// unknown lies outside the level holds zero (no sum ever writes another value
+// into it), and only whole fine cells past an odd edge have to be masked.  Bound
+// by load latency, so the 36 coefficients of a cell are loaded before any is
+// added; testing every coupling's bounds instead, with a straight-line path for
+// the interior beside it, serialised the loads:
+// 38-41 us, now 6.1 us (401 x 41 channel, FP64) and 7.2 us (12 caps, FP32).
+template <class T, int COMP>
+__device__ __forceinline__ void galc_cell(const CLevelT<T> &Fl, const CMember &fm, const CLevelT<T> &L, int J, int I,
+                                          long long pc) {
   const T *src = COMP == 0 ? Fl.cu : Fl.cv;
+  T v[4][9];
 #pragma unroll
-  for (int k = 0; k < 9; ++k) {
-    int cc, jj, i2;
-    slot_pos(COMP, k, DJ, DI, cc, jj, i2);  // offsets from the coarse cell's first fine cell
-    const int s = agg_slot(COMP, cc, jj >> 1, i2 >> 1);
-    if (s >= 0) cf[s] += (double)src[k * Fl.na + pf];
+  for (int q = 0; q < 4; ++q) {
+    const int j = 2 * J + (q >> 1), i = 2 * I + (q & 1);
+    const bool ok = cvalid(fm, COMP, j, i);
+    const long long pf = ok ? cp2(fm, j, i) : cp2(fm, 2 * J, 2 * I);
+#pragma unroll
+    for (int k = 0; k < 9; ++k) {
+      const T a = src[k * Fl.na + pf];
+      v[q][k] = ok ? a : (T)0.0;
+    }
   }
+  double cf[9] = {0, 0, 0, 0, 0, 0, 0, 0, 0};
+#pragma unroll
+  for (int q = 0; q < 4; ++q)
+#pragma unroll
+    for (int k = 0; k < 9; ++k) {
+      int cc, jj, i2;
+      slot_pos(COMP, k, q >> 1, q & 1, cc, jj, i2);  // offsets from the coarse cell's first fine cell
+      const int s = agg_slot(COMP, cc, jj >> 1, i2 >> 1);
+      if (s >= 0) cf[s] += (double)v[q][k];
+    }
+  T *dst = COMP == 0 ? L.cu : L.cv;
+#pragma unroll
+  for (int k = 0; k < 9; ++k) dst[k * L.na + pc] = (T)cf[k];
 }
 
-// level l (Fl) -> level l+1 (L), accumulated in FP64.  Away from the
-// level's edges (the test below: every fine cell and every unknown its row
-// reaches is valid) the sums run with constant slots, in the same order as
-// the general loop.
 template <class T>
 __global__ void __launch_bounds__(IMAU_WG) k_galc(CLevelT<T> Fl, CLevelT<T> L, const int *__restrict__ active) {
   CTILE_SETUP
@@ -352,48 +395,10 @@ __global__ void __launch_bounds__(IMAU_WG) k_galc(CLevelT<T> Fl, CLevelT<T> L, c
     const int I = t.i0 + ii;
     if (I >= cm.nx) break;
     const long long pc = cp2(cm, J, I);
-    const bool inner = J >= 1 && I >= 1;
-    const bool plain_u = inner && 2 * J + 2 < fm.nyu && 2 * I + 2 < fm.nxu && 2 * J + 1 < fm.nyv && 2 * I + 2 < fm.nxv;
-    const bool plain_v = inner && 2 * J + 2 < fm.nyv && 2 * I + 2 < fm.nxv && 2 * J + 2 < fm.nyu && 2 * I + 1 < fm.nxu;
-    if (plain_u && cvalid(cm, 0, J, I)) {
-      double cf[9] = {0, 0, 0, 0, 0, 0, 0, 0, 0};
-      galc_plain<T, 0, 0, 0>(Fl, fm, J, I, cf);
-      galc_plain<T, 0, 0, 1>(Fl, fm, J, I, cf);
-      galc_plain<T, 0, 1, 0>(Fl, fm, J, I, cf);
-      galc_plain<T, 0, 1, 1>(Fl, fm, J, I, cf);
-#pragma unroll
-      for (int k = 0; k < 9; ++k) L.cu[k * L.na + pc] = (T)cf[k];
-    }
-    if (plain_v && cvalid(cm, 1, J, I)) {
-      double cf[9] = {0, 0, 0, 0, 0, 0, 0, 0, 0};
-      galc_plain<T, 1, 0, 0>(Fl, fm, J, I, cf);
-      galc_plain<T, 1, 0, 1>(Fl, fm, J, I, cf);
-      galc_plain<T, 1, 1, 0>(Fl, fm, J, I, cf);
-      galc_plain<T, 1, 1, 1>(Fl, fm, J, I, cf);
-#pragma unroll
-      for (int k = 0; k < 9; ++k) L.cv[k * L.na + pc] = (T)cf[k];
-    }
-    for (int comp = 0; comp < 2; ++comp) {
-      if (!cvalid(cm, comp, J, I) || (comp == 0 ? plain_u : plain_v)) continue;
-      double cf[9] = {0, 0, 0, 0, 0, 0, 0, 0, 0};
-      const T *src = comp == 0 ? Fl.cu : Fl.cv;
-      for (int dj = 0; dj < 2; ++dj)
-        for (int di = 0; di < 2; ++di) {
-          const int j = 2 * J + dj, i = 2 * I + di;
-          if (!cvalid(fm, comp, j, i)) continue;
-          const long long pf = cp2(fm, j, i);
-#pragma unroll
-          for (int k = 0; k < 9; ++k) {
-            int cc, jj, i2;
-            slot_pos(comp, k, j, i, cc, jj, i2);
-            if (!cvalid(fm, cc, jj, i2)) continue;
-            const int s = agg_slot(comp, cc, (jj >> 1) - J, (i2 >> 1) - I);
-            if (s >= 0) cf[s] += (double)src[k * Fl.na + pf];
-          }
-        }
-      T *dst = comp == 0 ? L.cu : L.cv;
-#pragma unroll
-      for (int k = 0; k < 9; ++k) dst[k * L.na + pc] = (T)cf[k];
+    if (blockIdx.y == 0) {
+      if (cvalid(cm, 0, J, I)) galc_cell<T, 0>(Fl, fm, L, J, I, pc);
+    } else {
+      if (cvalid(cm, 1, J, I)) galc_cell<T, 1>(Fl, fm, L, J, I, pc);
     }
   }
 }
@@ -1049,12 +1054,12 @@ void setup_t(const imau::Launch &F, const KP &kp, const imau::Coef &c, const ima
   hipLaunchKernelGGL(kp0, dim3(L1.ntiles), wg(), 0, F.s, F.mem, kp, coef64(c), L1, act, P.plain);
   if (P.nlist > 0) {
     auto kg = kp.cross ? k_gal0_list<T, 1> : k_gal0_list<T, 0>;
-    hipLaunchKernelGGL(kg, dim3((P.nlist + 255) / 256), dim3(256), 0, F.s, F.mem, kp, coef64(c), L1, act, P.plain,
+    hipLaunchKernelGGL(kg, dim3((8 * P.nlist + 255) / 256), dim3(256), 0, F.s, F.mem, kp, coef64(c), L1, act, P.plain,
                        P.list, P.nlist);
   }
   for (size_t l = 1; l < P.levels.size(); ++l) {
     const CLevelT<T> Fl = view<T>(P, (int)l - 1), L = view<T>(P, (int)l);
-    hipLaunchKernelGGL(k_galc<T>, dim3(L.ntiles), wg(), 0, F.s, Fl, L, act);
+    hipLaunchKernelGGL(k_galc<T>, dim3(L.ntiles, 2), wg(), 0, F.s, Fl, L, act);
   }
 }
 
