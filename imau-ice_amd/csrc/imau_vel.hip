@@ -282,12 +282,18 @@ static void build_mg(imau_problem *P) {
     HIPCHK(hipMemcpy(lv->mem_d.p, lv->mem.data(), lv->mem.size() * sizeof(CMember), hipMemcpyHostToDevice));
     HIPCHK(hipMemcpy(lv->tiles_d.p, lv->tiles.data(), lv->tiles.size() * sizeof(Tile), hipMemcpyHostToDevice));
     P->plan.levels.push_back(imau::MGLevelDev{lv->mem_d.p, lv->tiles_d.p, (int)lv->tiles.size(), lev, off,
-                                              lv->data.p, false});
+                                              lv->data.p, false, 0});
     P->mg.push_back(std::move(lv));
   }
   P->mg_depth.alloc(P->ngrids);
   HIPCHK(hipMemcpy(P->mg_depth.p, depth.data(), P->ngrids * sizeof(int), hipMemcpyHostToDevice));
-  for (int d : depth) P->plan.levels[d - 1].ends = true;
+  for (int g = 0; g < P->ngrids; ++g) {
+    imau::MGLevelDev &lv = P->plan.levels[depth[g] - 1];
+    const CMember &c = P->mg[depth[g] - 1]->mem[g];
+    lv.ends = true;
+    // one thread per red-black pair of cells, whole wavefronts
+    lv.cthreads = std::max(lv.cthreads, (c.nx * ((c.ny + 1) / 2) + 63) / 64 * 64);
+  }
   P->plan.depth = P->mg_depth.p;
   P->plan.ngrids = P->ngrids;
   P->mg_plain.alloc((size_t)P->plan.levels[0].na);

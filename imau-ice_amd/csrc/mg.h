@@ -23,6 +23,7 @@ struct MGLevelDev {
   long long na;
   void *data;
   bool ends;  // some member's coarsest level is this one
+  int cthreads;  // threads of the workgroup that solves the largest such member
 };
 
 // FP32 copies of the fine-level coefficients and the FP32 right-hand side / iterate

@@ -655,69 +655,100 @@ __global__ void __launch_bounds__(IMAU_WG) k_cprolong(CLevelT<T> Fl, CLevelT<T> 
   }
 }
 
-// the coarsest level of each member: one 1024-thread workgroup, thread q owns
-// cell (J, I) = (q % ny, q / ny) with its u and v rows in registers and the
-// iterate in LDS; nsweeps symmetric four-colour Gauss-Seidel sweeps from zero
+// the coarsest level of each member: one workgroup, nsweeps symmetric
+// four-colour Gauss-Seidel sweeps from zero with the iterate in LDS.
+// Bound by the latency of its chain of colour phases (LDS reads, the row's sum,
+// a write, a barrier), so there are as few and as short phases as possible:
+//   - thread q owns the q-th red and the q-th black cell (u and v rows, in
+//     registers), so all lanes work in every phase and half as many waves meet
+//     at its barrier; the launch has only the threads that the level's largest
+//     member needs;
+//   - a colour updated twice in a row (the turning points of the symmetric
+//     sweeps) keeps its values, so it is updated once: 6 nsweeps + 1 phases for 8 nsweeps;
+//   - the rows are divided by their diagonal beforehand and summed in two
+//     halves, and a halo of zeros in LDS replaces the bounds tests.
+// 401 x 41 channel (26 x 3 cells, FP64): 19.8 -> 9.7 us; 12 caps of 96-512
+// cells (up to 32 x 32, FP32): 18.9 -> 12.2 us.
+constexpr int CL = IMAU_CMAX + 2;  // LDS row length, one-cell halo
+
+__device__ __forceinline__ float recip(float D) { return __builtin_amdgcn_rcpf(D); }
+__device__ __forceinline__ double recip(double D) { return 1.0 / D; }
+
+// a row divided by its diagonal: x = b - sum_k cf[k] x_k (zero where the diagonal is)
 template <class T>
-__device__ __forceinline__ void coarse_row_load(const CLevelT<T> &L, const CMember &m, int comp, int J, int I,
-                                                bool valid, T (&cf)[9], int (&nb)[9], T &b) {
-  const long long p = cp2(m, J, I);
-  const T *src = comp == 0 ? L.cu : L.cv;
-  b = valid ? (comp == 0 ? L.bu : L.bv)[p] : (T)0.0;
+struct CoarseRow {
+  T cf[8], b;
+  int l;       // LDS index, -1: no row
+  long long p;
+};
+
+template <class T, int COMP>
+__device__ __forceinline__ void coarse_row_load(const CLevelT<T> &L, const CMember &m, int J, int I, bool in,
+                                                CoarseRow<T> &r) {
+  r.l = -1;
+  if (!in || !cvalid(m, COMP, J, I)) return;
+  r.p = cp2(m, J, I);
+  const T *src = COMP == 0 ? L.cu : L.cv;
+  const T D = src[r.p], inv = D != (T)0.0 ? recip(D) : (T)0.0;
 #pragma unroll
-  for (int k = 0; k < 9; ++k) {
-    int cc, JJ, II;
-    slot_pos(comp, k, J, I, cc, JJ, II);
-    const bool ok = valid && (k == 0 || cvalid(m, cc, JJ, II));
-    cf[k] = ok ? src[k * L.na + p] : (T)0.0;
-    nb[k] = ok ? cc * (IMAU_CMAX * IMAU_CMAX) + II * m.ny + JJ : 0;
+  for (int k = 0; k < 8; ++k) r.cf[k] = src[(k + 1) * L.na + r.p] * inv;
+  r.b = (COMP == 0 ? L.bu : L.bv)[r.p] * inv;
+  r.l = (I + 1) * CL + J + 1;
+}
+
+template <class T, int COMP>
+__device__ __forceinline__ void coarse_row_gs(const CoarseRow<T> &r, T *su, T *sv) {
+  if (r.l < 0) return;
+  T s[2] = {r.b, (T)0.0};
+#pragma unroll
+  for (int k = 0; k < 8; ++k) {
+    int cc, dj, di;
+    slot_pos(COMP, k + 1, 0, 0, cc, dj, di);
+    s[k & 1] -= r.cf[k] * (cc == 0 ? su : sv)[r.l + di * CL + dj];
   }
+  (COMP == 0 ? su : sv)[r.l] = s[0] + s[1];
 }
 
 template <class T>
-__global__ void __launch_bounds__(1024) k_coarsest(CLevelT<T> L, const int *__restrict__ active, int nsweeps) {
-  __shared__ T sx[2 * IMAU_CMAX * IMAU_CMAX];
+__global__ void __launch_bounds__(IMAU_CMAX *IMAU_CMAX / 2) k_coarsest(CLevelT<T> L, const int *__restrict__ active,
+                                                                      int nsweeps) {
+  __shared__ T su[CL * CL], sv[CL * CL];
   const int g = blockIdx.x;
   if (!active[g] || L.depth[g] != L.lev) return;
   const CMember cm = L.mem[g];
-  const int n = cm.nx * cm.ny;
-  const int q = threadIdx.x;
-  const int J = q % cm.ny, I = q / cm.ny;
-  const bool in = q < n;
-  const bool vu = in && cvalid(cm, 0, J, I), vv = in && cvalid(cm, 1, J, I);
-  T cu[9], cv[9], bu, bv;
-  int nu[9], nv[9];
-  coarse_row_load(L, cm, 0, J, I, vu, cu, nu, bu);
-  coarse_row_load(L, cm, 1, J, I, vv, cv, nv, bv);
-  sx[q] = (T)0.0;
-  sx[IMAU_CMAX * IMAU_CMAX + q] = (T)0.0;
+  const int q = threadIdx.x, half = (cm.ny + 1) / 2, I = q / half, m = 2 * (q - I * half);
+  const bool in = I < cm.nx;
+  const int J0 = m + (I & 1), J1 = m + ((I + 1) & 1);  // red: I + J even
+  CoarseRow<T> u0, u1, v0, v1;
+  coarse_row_load<T, 0>(L, cm, J0, I, in, u0);
+  coarse_row_load<T, 0>(L, cm, J1, I, in, u1);
+  coarse_row_load<T, 1>(L, cm, J0, I, in, v0);
+  coarse_row_load<T, 1>(L, cm, J1, I, in, v1);
+  for (int k = q; k < CL * CL; k += blockDim.x) {
+    su[k] = (T)0.0;
+    sv[k] = (T)0.0;
+  }
   __syncthreads();
-  const int par = (I + J) & 1;
-  for (int sw = 0; sw < 2 * nsweeps; ++sw) {
-#pragma unroll
-    for (int q4 = 0; q4 < 4; ++q4) {
-      const int color = (sw & 1) ? 3 - q4 : q4;
-      if (par == (color & 1)) {
-        if (color < 2 && vu) {
-          T S = (T)0.0;
-#pragma unroll
-          for (int k = 1; k < 9; ++k) S += cu[k] * sx[nu[k]];
-          sx[q] = (cu[0] != (T)0.0) ? mdiv(bu - S, cu[0]) : (T)0.0;
-        } else if (color >= 2 && vv) {
-          T S = (T)0.0;
-#pragma unroll
-          for (int k = 1; k < 9; ++k) S += cv[k] * sx[nv[k]];
-          sx[IMAU_CMAX * IMAU_CMAX + q] = (cv[0] != (T)0.0) ? mdiv(bv - S, cv[0]) : (T)0.0;
-        }
-      }
-      __syncthreads();
-    }
+  coarse_row_gs<T, 0>(u0, su, sv);
+  __syncthreads();
+  for (int sw = 0; sw < nsweeps; ++sw) {
+    coarse_row_gs<T, 0>(u1, su, sv);
+    __syncthreads();
+    coarse_row_gs<T, 1>(v0, su, sv);
+    __syncthreads();
+    coarse_row_gs<T, 1>(v1, su, sv);
+    __syncthreads();
+    coarse_row_gs<T, 1>(v0, su, sv);
+    __syncthreads();
+    coarse_row_gs<T, 0>(u1, su, sv);
+    __syncthreads();
+    coarse_row_gs<T, 0>(u0, su, sv);
+    __syncthreads();
   }
-  if (in) {
-    const long long p = cp2(cm, J, I);
-    if (vu) L.xu[p] = sx[q];
-    if (vv) L.xv[p] = sx[IMAU_CMAX * IMAU_CMAX + q];
-  }
+  if (u0.l >= 0) L.xu[u0.p] = su[u0.l];
+  if (u1.l >= 0) L.xu[u1.p] = su[u1.l];
+  if (v0.l >= 0) L.xv[v0.p] = sv[v0.l];
+  if (v1.l >= 0) L.xv[v1.p] = sv[v1.l];
 }
 
 // ---------------------------------------------------------------------------
@@ -1071,7 +1102,7 @@ void coarse_t(hipStream_t s, const imau::MGPlan &P, const int *act) {
     const CLevelT<T> C = view<T>(P, l);
     fill<T>(s, C.xu, 2 * C.na);
     if (P.levels[l].ends)
-      hipLaunchKernelGGL(k_coarsest<T>, dim3(P.ngrids), dim3(1024), 0, s, C, act, P.coarsest_sweeps);
+      hipLaunchKernelGGL(k_coarsest<T>, dim3(P.ngrids), dim3(P.levels[l].cthreads), 0, s, C, act, P.coarsest_sweeps);
     if (l + 1 == nl) break;
     for (int col = 0; col < 4; ++col) hipLaunchKernelGGL(k_cgs<T>, dim3(C.ntiles), wg(), 0, s, C, col, act);
     const CLevelT<T> N = view<T>(P, l + 1);
@@ -1092,7 +1123,8 @@ void coarse_fused_t(hipStream_t s, const imau::MGPlan &P, const int *act) {
   for (int l = 0; l < nl; ++l) {
     const CLevelT<T> C = view<T>(P, l), C2 = view2<T>(P, l);
     if (P.levels[l].ends)
-      hipLaunchKernelGGL(k_coarsest<T>, dim3(P.ngrids), dim3(1024), 0, s, C2, act, P.coarsest_sweeps);
+      hipLaunchKernelGGL(k_coarsest<T>, dim3(P.ngrids), dim3(P.levels[l].cthreads), 0, s, C2, act,
+                         P.coarsest_sweeps);
     if (l + 1 == nl) break;
     hipLaunchKernelGGL(k_cdown<T>, dim3(C.ntiles), dim3(CTH), 0, s, C, view<T>(P, l + 1), act);
   }
