@@ -17,11 +17,10 @@
 #define IMAU_TI 8           // tile extent along i
 #define IMAU_WG_I 4         // wavefronts per workgroup along i
 #define IMAU_WG (IMAU_TJ * IMAU_WG_I)
-// fused smoother sweep: tiles of IMAU_FTI x IMAU_FTJ cells staged in LDS with a
-// recomputed halo of IMAU_FH cells (four colour phases + the boundary rows)
+// fused fine-level smoother sweeps: tiles of IMAU_FTI x IMAU_FTJ cells staged in
+// LDS with a recomputed halo
 #define IMAU_FTI 16
 #define IMAU_FTJ 64
-#define IMAU_FH 5
 // tile height of the 3D viscosity kernel (16 and 32 measured slower than 8 on
 // the 64-member ensemble: fewer workgroups in flight)
 #define IMAU_VTI 8

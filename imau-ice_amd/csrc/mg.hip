@@ -803,116 +803,275 @@ __global__ void __launch_bounds__(IMAU_WG) k_smooth0(const Member *__restrict__ 
   }
 }
 
-// One fused fine-level Gauss-Seidel sweep: the tile plus a halo of IMAU_FH
-// cells is staged in LDS from zin (zero when zin is null), the four colour
-// phases (u red, u black, v red, v black; reversed when reverse != 0) update
-// shrinking regions -- after phase p the values are exact up to IMAU_FH-1-p
-// cells beyond the tile, because each row couples only neighbours at distance
-// one -- and then the domain-boundary rows of the tile are set from their
-// sources (exact one cell beyond the tile).  The tile is written to zout, a
-// different buffer, so the result equals the one-launch-per-colour sweep
-// exactly.  Periodic boundary rows, whose sources lie across the domain, are
-// completed by a separate colour-4 pass of k_smooth0.
-#define FRI (IMAU_FTI + 2 * IMAU_FH)
-#define FRJ (IMAU_FTJ + 2 * IMAU_FH)
+// Fused fine-level sweeps, one launch each way.  A tile (IMAU_FTI x IMAU_FTJ)
+// plus a halo of H cells is held in LDS; the four colour phases (u red, u black,
+// v red, v black; reversed on the way up) update shrinking regions -- every row
+// couples only neighbours at distance one -- and then the 'infinite' and 'zero'
+// domain-boundary rows are set from their sources.
+//   k_fine_down: the sweep from zero (H = 6: exact two cells beyond the tile
+//     before the boundary rows, one after them), then the residual of the tile
+//     and its restriction to level 1;
+//   k_fine_up: the iterate plus the prolonged level 1, staged as the sum, and
+//     the reversed sweep (H = 5); the result in the working precision, or
+//     (TO = double) in FP64 for the Krylov solver.
+// The right-hand side is read in the Krylov solver's FP64.  The results equal
+// one launch per colour, k_restrict0 and k_prolong0.  Periodic boundary rows,
+// whose sources lie across the domain, are completed by a colour-4 pass of
+// k_smooth0, and the restriction then runs on its own (RESTRICT = false).
+//
+// Bound by load latency at small sizes and by the fine coefficients at large
+// ones.  A thread owns at most one row of every colour (FTH threads cover the
+// largest region), so the coefficients of its four rows are loaded at once
+// before the first barrier and the phases touch only LDS.  401 x 41 channel
+// (FP64): sweep 17.1 + restriction 11.5 us -> k_fine_down 10.9 us, prolongation
+// 4.6 + sweep 17.1 us -> k_fine_up 10.6 us; 12 caps of 96-512 cells (FP32):
+// conversion 8.0 + sweep 30.3 + restriction 23.5 -> 31.7 us, prolongation 10.8 +
+// sweep 30.3 + conversion 6.8 -> 34.1 us.
+#define FTH 1024
 
-template <class T>
+// the coefficients of one fine row held in registers, with the accessors the
+// rows of stencil.h read them through; (j, i) is the row's own position
+template <class T, int COMP, int CROSS>
+struct FRow {
+  T n0, n1, nb0, nbm, beta, ns;  // N_a on both sides, N_b on both sides, beta_eff, N on the row's own grid
+  T y;
+  int j, i, l;                   // l: LDS index of the cell, -1: no row
+  uint8_t rt;
+  bool in;                       // the cell lies in the tile
+  __device__ __forceinline__ T na(const Member &, int jj, int ii) const {
+    return (COMP == 0 ? ii == i : jj == j) ? n0 : n1;
+  }
+  __device__ __forceinline__ T nb(const Member &, int jj, int ii) const {
+    return (COMP == 0 ? jj == j : ii == i) ? nb0 : nbm;
+  }
+  __device__ __forceinline__ T bx(const Member &, int, int) const { return beta; }
+  __device__ __forceinline__ T by(const Member &, int, int) const { return beta; }
+  __device__ __forceinline__ T ncx(const Member &, int, int) const { return ns; }
+  __device__ __forceinline__ T ncy(const Member &, int, int) const { return ns; }
+};
+
+// row of phase region cell q (region half-width R around the tile, halo H)
+template <class T, int H, int R, int COLOR, int CROSS, class TY>
+__device__ __forceinline__ void frow_load(const Member &m, const CoefT<T> &c, const CVecT<TY> &y, const Tile &t, int q,
+                                          FRow<T, (COLOR >> 1), CROSS> &r) {
+  constexpr int RH = IMAU_FTJ / 2 + R, N = (IMAU_FTI + 2 * R) * RH, RJ = IMAU_FTJ + 2 * H, COMP = COLOR >> 1;
+  static_assert(N <= FTH, "one row of every colour per thread");
+  r.l = -1;
+  r.in = false;
+  if (q >= N) return;
+  const int ib = t.i0 - H, jb = t.j0 - H;
+  const int li = H - R + q / RH;
+  const int lj = H - R + 2 * (q % RH) + ((COLOR ^ (ib + li + jb + H - R)) & 1);
+  const int i = ib + li, j = jb + lj;
+  if (i < 0 || j < 0 || i >= m.nx - (COMP == 0) || j >= m.ny - (COMP == 1)) return;
+  const long long p = p2(m, j, i);
+  r.j = j;
+  r.i = i;
+  r.rt = COMP == 0 ? c.rt_u[p] : c.rt_v[p];
+  r.y = (T)(COMP == 0 ? y.u : y.v)[p];
+  r.n0 = c.Na[p];
+  r.n1 = c.Na[COMP == 0 ? p + m.ny : p + 1];
+  r.beta = (COMP == 0 ? c.bcx : c.bcy)[p];
+  if (CROSS) {
+    // the row of the domain's first line is a boundary row: its N_b is not used
+    r.nb0 = c.Nb[p];
+    r.nbm = c.Nb[COMP == 0 ? p - (j > 0) : p - (i > 0 ? m.ny : 0)];
+  } else {
+    r.ns = (COMP == 0 ? c.Ncx : c.Ncy)[p];
+  }
+  if (is_bnd(r.rt)) return;
+  r.l = li * RJ + lj;
+  r.in = li >= H && li < H + IMAU_FTI && lj >= H && lj < H + IMAU_FTJ;
+}
+
+template <class T, int RJ>
 struct LAccT {
   const T *base;  // LDS region, element (0,0) at global (ib, jb)
   int ib, jb;
-  __device__ __forceinline__ T operator()(int jj, int ii) const { return base[(ii - ib) * FRJ + (jj - jb)]; }
+  __device__ __forceinline__ T operator()(int jj, int ii) const { return base[(ii - ib) * RJ + (jj - jb)]; }
 };
 
-template <class T>
-__global__ void __launch_bounds__(IMAU_WG) k_smooth_fused(const Member *__restrict__ mem, const Tile *__restrict__ ftiles,
-                                                          const KP kp, const CoefT<T> c, CVecT<T> zin, VecT<T> zout,
-                                                          CVecT<T> y, int reverse, const int *__restrict__ active) {
-  __shared__ T su[FRI * FRJ], sv[FRI * FRJ];
+// the row's off-diagonal sum S and diagonal D at the LDS iterate
+template <class T, int COMP, int CROSS, class A>
+__device__ __forceinline__ void frow_sd(const Member &m, const KP &kp, const FRow<T, COMP, CROSS> &r, const A &U,
+                                        const A &V, T &S, T &D) {
+  if (COMP == 0) u_sd_x<CROSS, T>(m, kp, r, r.j, r.i, r.rt, U, V, S, D);
+  else v_sd_x<CROSS, T>(m, kp, r, r.j, r.i, r.rt, U, V, S, D);
+}
+template <class T, int COMP, int CROSS, class A>
+__device__ __forceinline__ void frow_gs(const Member &m, const KP &kp, const FRow<T, COMP, CROSS> &r, const A &U,
+                                        const A &V, T *x) {
+  if (r.l < 0) return;
+  T S, D;
+  frow_sd<T, COMP, CROSS>(m, kp, r, U, V, S, D);
+  x[r.l] = mdiv(r.y - S, D);
+}
+
+// 'infinite' and 'zero' domain-boundary rows of the tile and E cells beyond it
+template <class T, int H, int E, class TY, class A>
+__device__ __forceinline__ void fine_boundary(const Member &m, const CoefT<T> &c, const CVecT<TY> &y, const Tile &t,
+                                              int tid, const A &U, const A &V, T *su, T *sv) {
+  constexpr int RJ = IMAU_FTJ + 2 * H, BJ = IMAU_FTJ + 2 * E, BI = IMAU_FTI + 2 * E;
+  for (int q = tid; q < BI * BJ; q += FTH) {
+    const int li = H - E + q / BJ, lj = H - E + q % BJ;
+    const int i = t.i0 - H + li, j = t.j0 - H + lj;
+    if (i < 0 || j < 0 || i >= m.nx || j >= m.ny) continue;
+    // rows of the domain's edges only (u: i = 0, nx-2, j = 0, ny-1; v likewise)
+    if (i > 0 && j > 0 && i < m.nx - 2 && j < m.ny - 2) continue;
+    const long long p = p2(m, j, i);
+    int jo, io;
+    if (i < m.nx - 1) {
+      const uint8_t rt = c.rt_u[p];
+      if (rt == RT_BND_ZERO || rt == RT_BND_INF) {
+        T val = (T)y.u[p];
+        if (rt == RT_BND_INF) {
+          bnd_src(rt, i, j, m.nx - 2, m.ny - 1, jo, io);
+          val += U(jo, io);
+        }
+        su[li * RJ + lj] = val;
+      }
+    }
+    if (j < m.ny - 1) {
+      const uint8_t rt = c.rt_v[p];
+      if (rt == RT_BND_ZERO || rt == RT_BND_INF) {
+        T val = (T)y.v[p];
+        if (rt == RT_BND_INF) {
+          bnd_src(rt, i, j, m.nx - 1, m.ny - 2, jo, io);
+          val += V(jo, io);
+        }
+        sv[li * RJ + lj] = val;
+      }
+    }
+  }
+}
+// whether the tile and E cells beyond it reach the domain's edges
+__device__ __forceinline__ bool at_edge(const Member &m, const Tile &t, int E) {
+  return t.i0 <= E || t.j0 <= E || t.i0 + IMAU_FTI + E > m.nx - 2 || t.j0 + IMAU_FTJ + E > m.ny - 2;
+}
+
+template <class T, int CROSS, bool RESTRICT, class TY>
+__global__ void __launch_bounds__(FTH) k_fine_down(const Member *__restrict__ mem, const Tile *__restrict__ ftiles,
+                                                   const KP kp, const CoefT<T> c, CVecT<TY> y, VecT<T> zout,
+                                                   CLevelT<T> N, const int *__restrict__ active) {
+  constexpr int H = 6, RI = IMAU_FTI + 2 * H, RJ = IMAU_FTJ + 2 * H;
+  __shared__ T su[RI * RJ], sv[RI * RJ], sr[2][IMAU_FTI * IMAU_FTJ];
   const Tile t = ftiles[imau_xcd_tile()];
   if (!active[t.g]) return;
   const Member m = mem[t.g];
-  const int nx = m.nx, ny = m.ny;
-  const int ib = t.i0 - IMAU_FH, jb = t.j0 - IMAU_FH;
-  const int tid = threadIdx.y * IMAU_TJ + threadIdx.x;
-  for (int q = tid; q < FRI * FRJ; q += IMAU_WG) {
-    const int li = q / FRJ, lj = q - li * FRJ;
-    const int i = ib + li, j = jb + lj;
-    T u = (T)0.0, v = (T)0.0;
-    if (zin.u && i >= 0 && j >= 0 && i < nx && j < ny) {
+  const int tid = threadIdx.x;
+  FRow<T, 0, CROSS> r0, r1;
+  FRow<T, 1, CROSS> r2, r3;
+  frow_load<T, H, 5, 0, CROSS>(m, c, y, t, tid, r0);
+  frow_load<T, H, 4, 1, CROSS>(m, c, y, t, tid, r1);
+  frow_load<T, H, 3, 2, CROSS>(m, c, y, t, tid, r2);
+  frow_load<T, H, 2, 3, CROSS>(m, c, y, t, tid, r3);
+  for (int q = tid; q < RI * RJ; q += FTH) {
+    su[q] = (T)0.0;
+    sv[q] = (T)0.0;
+  }
+  sr[0][tid] = (T)0.0;
+  sr[1][tid] = (T)0.0;
+  static_assert(IMAU_FTI * IMAU_FTJ == FTH, "one tile cell per thread");
+  __syncthreads();
+  const LAccT<T, RJ> U{su, t.i0 - H, t.j0 - H}, V{sv, t.i0 - H, t.j0 - H};
+  frow_gs<T, 0, CROSS>(m, kp, r0, U, V, su);
+  __syncthreads();
+  frow_gs<T, 0, CROSS>(m, kp, r1, U, V, su);
+  __syncthreads();
+  frow_gs<T, 1, CROSS>(m, kp, r2, U, V, sv);
+  __syncthreads();
+  frow_gs<T, 1, CROSS>(m, kp, r3, U, V, sv);
+  __syncthreads();
+  if (at_edge(m, t, 1)) {  // the same for the whole workgroup
+    fine_boundary<T, H, 1>(m, c, y, t, tid, U, V, su, sv);
+    __syncthreads();
+  }
+  {
+    const int li = tid / IMAU_FTJ, lj = tid % IMAU_FTJ, i = t.i0 + li, j = t.j0 + lj;
+    if (i < m.nx && j < m.ny) {
       const long long p = p2(m, j, i);
-      if (i < nx - 1) u = zin.u[p];
-      if (j < ny - 1) v = zin.v[p];
+      if (i < m.nx - 1) zout.u[p] = su[(li + H) * RJ + lj + H];
+      if (j < m.ny - 1) zout.v[p] = sv[(li + H) * RJ + lj + H];
+    }
+  }
+  if (!RESTRICT) return;
+  auto res = [&](const auto &r, const T *x, T *out) {
+    if (!r.in || !in_row(r.rt)) return;
+    T S, D;
+    frow_sd(m, kp, r, U, V, S, D);
+    out[(r.i - t.i0) * IMAU_FTJ + r.j - t.j0] = r.y - S - D * x[r.l];
+  };
+  res(r0, su, sr[0]);
+  res(r1, su, sr[0]);
+  res(r2, sv, sr[1]);
+  res(r3, sv, sr[1]);
+  __syncthreads();
+  const CMember nm = N.mem[t.g];
+  if (tid < 2 * (IMAU_FTI / 2) * (IMAU_FTJ / 2)) {
+    const int comp = tid / ((IMAU_FTI / 2) * (IMAU_FTJ / 2)), q = tid % ((IMAU_FTI / 2) * (IMAU_FTJ / 2));
+    const int li = q / (IMAU_FTJ / 2), lj = q % (IMAU_FTJ / 2), I = t.i0 / 2 + li, J = t.j0 / 2 + lj;
+    if (cvalid(nm, comp, J, I)) {
+      const T *s = sr[comp] + 2 * li * IMAU_FTJ + 2 * lj;
+      (comp == 0 ? N.bu : N.bv)[cp2(nm, J, I)] = (((s[0] + s[IMAU_FTJ]) + s[1]) + s[IMAU_FTJ + 1]);
+    }
+  }
+}
+
+// za: the pre-smoothed iterate; N.xu / N.xv: level 1's result
+template <class T, int CROSS, class TY, class TO>
+__global__ void __launch_bounds__(FTH) k_fine_up(const Member *__restrict__ mem, const Tile *__restrict__ ftiles,
+                                                 const KP kp, const CoefT<T> c, CVecT<TY> y, CVecT<T> za, VecT<TO> zout,
+                                                 CLevelT<T> N, const int *__restrict__ active) {
+  constexpr int H = 5, RI = IMAU_FTI + 2 * H, RJ = IMAU_FTJ + 2 * H;
+  __shared__ T su[RI * RJ], sv[RI * RJ];
+  const Tile t = ftiles[imau_xcd_tile()];
+  if (!active[t.g]) return;
+  const Member m = mem[t.g];
+  const CMember nm = N.mem[t.g];
+  const int tid = threadIdx.x;
+  FRow<T, 1, CROSS> r0, r1;
+  FRow<T, 0, CROSS> r2, r3;
+  frow_load<T, H, 4, 3, CROSS>(m, c, y, t, tid, r0);
+  frow_load<T, H, 3, 2, CROSS>(m, c, y, t, tid, r1);
+  frow_load<T, H, 2, 1, CROSS>(m, c, y, t, tid, r2);
+  frow_load<T, H, 1, 0, CROSS>(m, c, y, t, tid, r3);
+  for (int q = tid; q < RI * RJ; q += FTH) {
+    const int i = t.i0 - H + q / RJ, j = t.j0 - H + q % RJ;
+    T u = (T)0.0, v = (T)0.0;
+    if (i >= 0 && j >= 0 && i < m.nx && j < m.ny) {
+      const long long p = p2(m, j, i);
+      int Jc, Ic;
+      if (i < m.nx - 1) {
+        u = za.u[p];
+        if (fine_agg(m, c.rt_u, c.rt_v, 0, j, i, Jc, Ic)) u += N.xu[cp2(nm, Jc, Ic)];
+      }
+      if (j < m.ny - 1) {
+        v = za.v[p];
+        if (fine_agg(m, c.rt_u, c.rt_v, 1, j, i, Jc, Ic)) v += N.xv[cp2(nm, Jc, Ic)];
+      }
     }
     su[q] = u;
     sv[q] = v;
   }
   __syncthreads();
-  const LAccT<T> U{su, ib, jb}, V{sv, ib, jb};
-  for (int ph = 0; ph < 4; ++ph) {
-    const int color = reverse ? 3 - ph : ph;
-    const bool isu = color < 2;
-    const int r = IMAU_FH - 1 - ph;
-    const int li0 = IMAU_FH - r, lj0 = IMAU_FH - r;
-    // the region has an even width, so every row holds RW / 2 cells of this
-    // colour: lanes take those cells only (cells of one colour do not couple,
-    // so the order is free)
-    const int RW = IMAU_FTJ + 2 * r, RH = RW / 2, n = (IMAU_FTI + 2 * r) * RH;
-    for (int q = tid; q < n; q += IMAU_WG) {
-      const int li = li0 + q / RH;
-      const int lj = lj0 + 2 * (q % RH) + ((color ^ (ib + li + jb + lj0)) & 1);
-      const int i = ib + li, j = jb + lj;
-      if (i < 0 || j < 0 || i >= nx || j >= ny) continue;
-      if (isu && i >= nx - 1) continue;
-      if (!isu && j >= ny - 1) continue;
-      const long long p = p2(m, j, i);
-      const uint8_t rt = isu ? c.rt_u[p] : c.rt_v[p];
-      if (is_bnd(rt)) continue;
-      T S, D;
-      if (isu) u_sd<T>(m, kp, c, j, i, rt, U, V, S, D);
-      else v_sd<T>(m, kp, c, j, i, rt, U, V, S, D);
-      (isu ? su : sv)[li * FRJ + lj] = mdiv((isu ? y.u : y.v)[p] - S, D);
-    }
+  const LAccT<T, RJ> U{su, t.i0 - H, t.j0 - H}, V{sv, t.i0 - H, t.j0 - H};
+  frow_gs<T, 1, CROSS>(m, kp, r0, U, V, sv);
+  __syncthreads();
+  frow_gs<T, 1, CROSS>(m, kp, r1, U, V, sv);
+  __syncthreads();
+  frow_gs<T, 0, CROSS>(m, kp, r2, U, V, su);
+  __syncthreads();
+  frow_gs<T, 0, CROSS>(m, kp, r3, U, V, su);
+  __syncthreads();
+  if (at_edge(m, t, 0)) {  // the same for the whole workgroup
+    fine_boundary<T, H, 0>(m, c, y, t, tid, U, V, su, sv);
     __syncthreads();
   }
-  // domain-boundary rows of the tile ('infinite' and 'zero'; sources are interior rows)
-  for (int q = tid; q < IMAU_FTI * IMAU_FTJ; q += IMAU_WG) {
-    const int li = IMAU_FH + q / IMAU_FTJ, lj = IMAU_FH + q % IMAU_FTJ;
-    const int i = ib + li, j = jb + lj;
-    if (i >= nx || j >= ny) continue;
+  const int li = tid / IMAU_FTJ, lj = tid % IMAU_FTJ, i = t.i0 + li, j = t.j0 + lj;
+  if (i < m.nx && j < m.ny) {
     const long long p = p2(m, j, i);
-    if (i < nx - 1) {
-      const uint8_t rt = c.rt_u[p];
-      if (rt == RT_BND_ZERO || rt == RT_BND_INF) {
-        T val = y.u[p];
-        if (rt == RT_BND_INF) {
-          int jo, io;
-          bnd_src(rt, i, j, nx - 2, ny - 1, jo, io);
-          val += U(jo, io);
-        }
-        su[li * FRJ + lj] = val;
-      }
-    }
-    if (j < ny - 1) {
-      const uint8_t rt = c.rt_v[p];
-      if (rt == RT_BND_ZERO || rt == RT_BND_INF) {
-        T val = y.v[p];
-        if (rt == RT_BND_INF) {
-          int jo, io;
-          bnd_src(rt, i, j, nx - 1, ny - 2, jo, io);
-          val += V(jo, io);
-        }
-        sv[li * FRJ + lj] = val;
-      }
-    }
-  }
-  __syncthreads();
-  for (int q = tid; q < IMAU_FTI * IMAU_FTJ; q += IMAU_WG) {
-    const int li = IMAU_FH + q / IMAU_FTJ, lj = IMAU_FH + q % IMAU_FTJ;
-    const int i = ib + li, j = jb + lj;
-    if (i >= nx || j >= ny) continue;
-    const long long p = p2(m, j, i);
-    if (i < nx - 1) zout.u[p] = su[li * FRJ + lj];
-    if (j < ny - 1) zout.v[p] = sv[li * FRJ + lj];
+    if (i < m.nx - 1) zout.u[p] = (TO)su[(li + H) * RJ + lj + H];
+    if (j < m.ny - 1) zout.v[p] = (TO)sv[(li + H) * RJ + lj + H];
   }
 }
 
@@ -1154,27 +1313,36 @@ void vcycle_t(const imau::Launch &F, const KP &kp, const CoefT<T> &cf, const ima
   hipLaunchKernelGGL(k_smooth0<T>, dim3(F.ntiles), wg(), 0, s, F.mem, F.tiles, kp, cf, z, y, 4, act);
 }
 
-// fused sweeps: pre-smoothing from zero into za, post-smoothing from za into zb
-template <class T>
-void vcycle_fused_t(const imau::Launch &F, const KP &kp, const CoefT<T> &cf, const imau::MGPlan &P, CVecT<T> y,
-                    VecT<T> za, VecT<T> zb, const int *act, imau::MGMark mark, void *mctx) {
+// fused sweeps: pre-smoothing from zero into za, post-smoothing from za into
+// z (FP64).  With periodic boundaries, whose rows need a pass of their own on
+// the working-precision iterate, the restriction runs on its own and the
+// post-smoothed iterate goes through zb; yt is then the right-hand side in
+// the working precision (null otherwise).
+template <class T, int CROSS>
+void vcycle_fused_t(const imau::Launch &F, const KP &kp, const CoefT<T> &cf, const imau::MGPlan &P, CVecT<double> y,
+                    CVecT<T> yt, VecT<T> za, VecT<T> zb, VecT<double> z, const int *act, imau::MGMark mark, void *mctx) {
   hipStream_t s = F.s;
-  if (mark) mark(mctx, 0);
-  hipLaunchKernelGGL(k_smooth_fused<T>, dim3(P.nftiles), wg(), 0, s, F.mem, P.ftiles, kp, cf, CVecT<T>{nullptr, nullptr},
-                     za, y, 0, act);
-  if (P.periodic)
-    hipLaunchKernelGGL(k_smooth0<T>, dim3(F.ntiles), wg(), 0, s, F.mem, F.tiles, kp, cf, za, y, 4, act);
-  if (mark) mark(mctx, 1);
   const CLevelT<T> L1 = view<T>(P, 0);
-  auto kr = kp.cross ? k_restrict0<T, 1> : k_restrict0<T, 0>;
-  hipLaunchKernelGGL(kr, dim3(L1.ntiles), wg(), 0, s, F.mem, kp, cf, y, CVecT<T>{za.u, za.v}, L1, act);
+  const CVecT<T> zac{za.u, za.v};
+  if (mark) mark(mctx, 0);
+  if (!P.periodic) {
+    hipLaunchKernelGGL((k_fine_down<T, CROSS, true, double>), dim3(P.nftiles), dim3(FTH), 0, s, F.mem, P.ftiles, kp, cf,
+                       y, za, L1, act);
+    if (mark) mark(mctx, 1);
+    coarse_fused_t<T>(s, P, act);
+    hipLaunchKernelGGL((k_fine_up<T, CROSS, double, double>), dim3(P.nftiles), dim3(FTH), 0, s, F.mem, P.ftiles, kp, cf,
+                       y, zac, z, view2<T>(P, 0), act);
+    return;
+  }
+  hipLaunchKernelGGL((k_fine_down<T, CROSS, false, double>), dim3(P.nftiles), dim3(FTH), 0, s, F.mem, P.ftiles, kp, cf, y,
+                     za, L1, act);
+  hipLaunchKernelGGL(k_smooth0<T>, dim3(F.ntiles), wg(), 0, s, F.mem, F.tiles, kp, cf, za, yt, 4, act);
+  if (mark) mark(mctx, 1);
+  hipLaunchKernelGGL((k_restrict0<T, CROSS>), dim3(L1.ntiles), wg(), 0, s, F.mem, kp, cf, yt, zac, L1, act);
   coarse_fused_t<T>(s, P, act);
-  hipLaunchKernelGGL(k_prolong0<T>, dim3(F.ntiles), wg(), 0, s, F.mem, F.tiles, cf.rt_u, cf.rt_v, za, view2<T>(P, 0),
-                     act);
-  hipLaunchKernelGGL(k_smooth_fused<T>, dim3(P.nftiles), wg(), 0, s, F.mem, P.ftiles, kp, cf, CVecT<T>{za.u, za.v},
-                     zb, y, 1, act);
-  if (P.periodic)
-    hipLaunchKernelGGL(k_smooth0<T>, dim3(F.ntiles), wg(), 0, s, F.mem, F.tiles, kp, cf, zb, y, 4, act);
+  hipLaunchKernelGGL((k_fine_up<T, CROSS, double, T>), dim3(P.nftiles), dim3(FTH), 0, s, F.mem, P.ftiles, kp, cf, y, zac,
+                     zb, view2<T>(P, 0), act);
+  hipLaunchKernelGGL(k_smooth0<T>, dim3(F.ntiles), wg(), 0, s, F.mem, F.tiles, kp, cf, zb, yt, 4, act);
 }
 
 }  // namespace
@@ -1202,27 +1370,32 @@ void mg_setup(const Launch &F, const KP &kp, const Coef &c, const MGPlan &P, boo
 
 void mg_vcycle(const Launch &F, const KP &kp, const Coef &c, const MGPlan &P, bool fp32, const double *yu,
                const double *yv, double *zu, double *zv, const int *active, MGMark mark, void *mark_ctx) {
+  const CVecT<double> y{yu, yv};
+  const VecT<double> z{zu, zv};
   if (fp32) {
-    VecT<float> y32{P.f32.yu, P.f32.yv}, z32{P.f32.zu, P.f32.zv}, z32b{P.f32.zu2, P.f32.zv2};
-    hipLaunchKernelGGL(k_prep<float>, dim3(F.ntiles), wg(), 0, F.s, F.mem, F.tiles, CVecT<double>{yu, yv}, y32, z32,
-                       active);
+    const VecT<float> y32{P.f32.yu, P.f32.yv}, z32{P.f32.zu, P.f32.zv}, z32b{P.f32.zu2, P.f32.zv2};
+    const CVecT<float> y32c{y32.u, y32.v};
     const CoefT<float> cf = coef32(P.f32, c);
+    const bool own = !P.fused || P.periodic;  // paths on an FP32 right-hand side and result
+    if (own)
+      hipLaunchKernelGGL(k_prep<float>, dim3(F.ntiles), wg(), 0, F.s, F.mem, F.tiles, y, y32, z32, active);
     if (P.fused) {
-      vcycle_fused_t<float>(F, kp, cf, P, CVecT<float>{y32.u, y32.v}, z32, z32b, active, mark, mark_ctx);
-      z32 = z32b;
+      auto run = kp.cross ? vcycle_fused_t<float, 1> : vcycle_fused_t<float, 0>;
+      run(F, kp, cf, P, y, y32c, z32, z32b, z, active, mark, mark_ctx);
     } else {
-      vcycle_t<float>(F, kp, cf, P, CVecT<float>{y32.u, y32.v}, z32, active, mark, mark_ctx);
+      vcycle_t<float>(F, kp, cf, P, y32c, z32, active, mark, mark_ctx);
     }
-    hipLaunchKernelGGL(k_fin, dim3(F.ntiles), wg(), 0, F.s, F.mem, F.tiles, CVecT<float>{z32.u, z32.v},
-                       VecT<double>{zu, zv}, active);
+    if (own) {
+      const VecT<float> r = P.fused ? z32b : z32;
+      hipLaunchKernelGGL(k_fin, dim3(F.ntiles), wg(), 0, F.s, F.mem, F.tiles, CVecT<float>{r.u, r.v}, z, active);
+    }
   } else if (P.fused) {
-    vcycle_fused_t<double>(F, kp, coef64(c), P, CVecT<double>{yu, yv}, VecT<double>{P.zu64, P.zv64},
-                           VecT<double>{zu, zv}, active, mark, mark_ctx);
+    auto run = kp.cross ? vcycle_fused_t<double, 1> : vcycle_fused_t<double, 0>;
+    run(F, kp, coef64(c), P, y, y, VecT<double>{P.zu64, P.zv64}, z, z, active, mark, mark_ctx);
   } else {
-    VecT<double> z{zu, zv};
-    hipLaunchKernelGGL(k_prep<double>, dim3(F.ntiles), wg(), 0, F.s, F.mem, F.tiles, CVecT<double>{yu, yv},
-                       VecT<double>{nullptr, nullptr}, z, active);
-    vcycle_t<double>(F, kp, coef64(c), P, CVecT<double>{yu, yv}, z, active, mark, mark_ctx);
+    hipLaunchKernelGGL(k_prep<double>, dim3(F.ntiles), wg(), 0, F.s, F.mem, F.tiles, y, VecT<double>{nullptr, nullptr}, z,
+                       active);
+    vcycle_t<double>(F, kp, coef64(c), P, y, z, active, mark, mark_ctx);
   }
 }
 
