@@ -15,6 +15,8 @@
   const int j = t.j0 + (int)threadIdx.x;
 
 #define FOR_TILE_ROWS for (int ii = threadIdx.y; ii < IMAU_TI; ii += IMAU_WG_I)
+// one cell at a time, where unrolling would cost more registers than it hides latency
+#define FOR_TILE_ROWS_1 _Pragma("unroll 1") for (int ii = threadIdx.y; ii < IMAU_TI; ii += IMAU_WG_I)
 #define FOR_VTILE_ROWS _Pragma("unroll 1") for (int ii = threadIdx.y; ii < IMAU_VTI; ii += IMAU_WG_I)
 
 // ---------------------------------------------------------------------------
@@ -921,8 +923,86 @@ __device__ __forceinline__ void v_row(const Member &m, const KP &kp, const CoefP
 
 
 
-#undef su
-#undef sv
+// The rows of one cell at the vectors (xu, xv): S and D of its u and v unknown,
+// from the loaded neighbourhood; only 'infinite' and 'periodic' boundary rows
+// read one more value, their source.
+__device__ __forceinline__ bool zero_row(uint8_t rt) { return rt == RT_ZERO || rt == RT_BND_ZERO; }
+__device__ __forceinline__ bool copy_row(uint8_t rt) { return rt == RT_BND_INF || rt == RT_BND_PER; }
+template <int CROSS>
+struct CellRows {
+  Hood<double> U, V;
+  HoodCoef<double> k;
+  uint8_t ru, rv;
+  __device__ __forceinline__ bool hu(const Member &m) const { return k.i < m.nx - 1; }  // the cell has a u unknown
+  __device__ __forceinline__ bool hv(const Member &m) const { return k.j < m.ny - 1; }
+  __device__ __forceinline__ void load(const Member &m, const CoefP &c, const double *xu, const double *xv, int j,
+                                       int i) {
+    const uint32_t p = (uint32_t)i * (uint32_t)m.ny + (uint32_t)j;
+    ru = (c.rt_u + m.off)[p];
+    rv = (c.rt_v + m.off)[p];
+    hood_load<double, CROSS>(m, c, xu, xv, j, i, U, V, k);
+  }
+  // the source of a boundary row that copies one
+  __device__ __forceinline__ long long u_src(const Member &m) const {
+    int jo, io;
+    bnd_src(ru, k.i, k.j, m.nx - 2, m.ny - 1, jo, io);
+    return p2(m, jo, io);
+  }
+  __device__ __forceinline__ long long v_src(const Member &m) const {
+    int jo, io;
+    bnd_src(rv, k.i, k.j, m.nx - 1, m.ny - 2, jo, io);
+    return p2(m, jo, io);
+  }
+  // interior and calving-front rows
+  __device__ __forceinline__ void u_in(const Member &m, const KP &kp, double &S, double &D) const {
+    u_sd_x<CROSS, double>(m, kp, k, k.j, k.i, ru, U, V, S, D);
+  }
+  __device__ __forceinline__ void v_in(const Member &m, const KP &kp, double &S, double &D) const {
+    v_sd_x<CROSS, double>(m, kp, k, k.j, k.i, rv, U, V, S, D);
+  }
+  __device__ __forceinline__ void u_sd(const Member &m, const KP &kp, const double *xu, double &S, double &D) const {
+    if (in_row(ru)) { u_in(m, kp, S, D); return; }
+    S = copy_row(ru) ? -xu[u_src(m)] : 0.0;
+    D = 1.0;
+  }
+  __device__ __forceinline__ void v_sd(const Member &m, const KP &kp, const double *xv, double &S, double &D) const {
+    if (in_row(rv)) { v_in(m, kp, S, D); return; }
+    S = copy_row(rv) ? -xv[v_src(m)] : 0.0;
+    D = 1.0;
+  }
+};
+// right-hand sides of the rows (tau: the driving stress at the row; ns: N on its
+// own grid, in the form without cross terms)
+template <int CROSS>
+__device__ __forceinline__ double u_rhs(const Member &m, const CoefP &c, int j, int i, uint8_t rt, double tau,
+                                        double ns) {
+  if (rt == RT_FREE) {
+    const double b = -tau * (m.dx * m.dx);
+    return CROSS ? b : b / ns;
+  }
+  if (rt == RT_MARGIN_I || rt == RT_MARGIN_O) return c.frhs[p2(m, j, (rt == RT_MARGIN_I) ? i : i + 1)];
+  return 0.0;
+}
+template <int CROSS>
+__device__ __forceinline__ double v_rhs(const Member &m, const CoefP &c, int j, int i, uint8_t rt, double tau,
+                                        double ns) {
+  if (rt == RT_FREE) {
+    const double b = -tau * (m.dx * m.dx);
+    return CROSS ? b : b / ns;
+  }
+  if (rt == RT_MARGIN_I || rt == RT_MARGIN_O) return c.frhs[p2(m, (rt == RT_MARGIN_I) ? j : j + 1, i)];
+  return 0.0;
+}
+// The operator kernels (k_apply, k_resid, k_bicg_init) are bound
+// by load latency at small sizes and by how many loads are in flight at large
+// ones: the some 25 values of a cell are all loaded before its rows are
+// evaluated.  (Both of a thread's cells at once took more registers than the
+// extra loads in flight were worth.)  k_apply 7.0 -> 5.1 us on the 401x41
+// channel (FP64), 23.4 -> 18.8 on 12 ice caps of 96 to 512 a side
+// (FP32 operator), k_bicg_init 9.6 -> 6.2, k_resid 6.7 -> 5.6.  k_resid_init
+// keeps its look-ups: loaded first it took 54 instead of 70 us on the 12 caps,
+// but 30 instead of 27 on 8 of 256x256.
+constexpr int TROWS = IMAU_TI / IMAU_WG_I;
 
 // ---------------------------------------------------------------------------
 // Picard step 3 (after the linear solve): velocity limits (:1432-1498),
@@ -1222,28 +1302,32 @@ __global__ void __launch_bounds__(IMAU_WG) k_net_warm(const Member *__restrict__
 
 // FP64 residual partial sums: sum (S + D x - b)^2 and sum b^2 over every row
 // of the system assembled at the current coefficients.
+template <int CROSS>
 __global__ void __launch_bounds__(IMAU_WG) k_resid(const Member *__restrict__ mem, const Tile *__restrict__ tiles,
                                                    const KP kp, const CoefP c, const double *__restrict__ xu,
                                                    const double *__restrict__ xv, double *__restrict__ partial) {
   TILE_SETUP
   double acc[2] = {0.0, 0.0};
-  const int nx = m.nx, ny = m.ny;
-  const GAcc U{xu, m}, V{xv, m};
-  if (j < ny) {
-    FOR_TILE_ROWS {
+  if (j < m.ny) {
+    FOR_TILE_ROWS_1 {
       const int i = t.i0 + ii;
-      if (i >= nx) break;
-      const long long p = p2(m, j, i);
-      double S, D, b;
-      if (i < nx - 1) {
-        u_row(m, kp, c, j, i, c.rt_u[p], U, V, S, D, b);
-        const double r = S + D * xu[p] - b;
+      if (i >= m.nx) break;
+      CellRows<CROSS> cr;
+      cr.load(m, c, xu, xv, j, i);
+      const double tu = c.taudx[p2(m, j, i)];
+      const double tv = c.taudy[p2(m, j, i)];
+      double S, D;
+      if (cr.hu(m)) {
+        cr.u_sd(m, kp, xu, S, D);
+        const double b = u_rhs<CROSS>(m, c, j, i, cr.ru, tu, cr.k.nb0);
+        const double r = S + D * cr.U.c - b;
         acc[0] += r * r;
         acc[1] += b * b;
       }
-      if (j < ny - 1) {
-        v_row(m, kp, c, j, i, c.rt_v[p], U, V, S, D, b);
-        const double r = S + D * xv[p] - b;
+      if (cr.hv(m)) {
+        cr.v_sd(m, kp, xv, S, D);
+        const double b = v_rhs<CROSS>(m, c, j, i, cr.rv, tv, cr.k.nbw);
+        const double r = S + D * cr.V.c - b;
         acc[0] += r * r;
         acc[1] += b * b;
       }
@@ -1813,7 +1897,8 @@ void post(const Launch &L, const KP &kp, const Fields &f, const double *xu, cons
                      relax, mix);
 }
 void resid(const Launch &L, const KP &kp, const Coef &c, const double *xu, const double *xv, double *partial) {
-  hipLaunchKernelGGL(k_resid, dim3(L.ntiles), wg(), 0, L.s, L.mem, L.tiles, kp, to_p(c), xu, xv, partial);
+  auto k = kp.cross ? k_resid<1> : k_resid<0>;
+  hipLaunchKernelGGL(k, dim3(L.ntiles), wg(), 0, L.s, L.mem, L.tiles, kp, to_p(c), xu, xv, partial);
 }
 void member_sum3(hipStream_t s, int ngrids, const int *tstart, const double *partial, double *out) {
   hipLaunchKernelGGL(k_member_sum<3>, dim3(ngrids), dim3(256), 0, s, tstart, partial, out);
@@ -1905,24 +1990,29 @@ __global__ void __launch_bounds__(IMAU_WG) k_apply(const Member *__restrict__ me
                                                    const int *__restrict__ active, double *__restrict__ partial) {
   TILE_SETUP
   double acc[2] = {0.0, 0.0};
-  const GAcc U{x.u, m}, V{x.v, m};
   if (j < m.ny && active[t.g]) {
-    FOR_TILE_ROWS {
+    FOR_TILE_ROWS_1 {
       const int i = t.i0 + ii;
       if (i >= m.nx) break;
+      CellRows<CROSS> cr;
+      cr.load(m, c, x.u, x.v, j, i);
+      const double wu = w.u ? w.u[p2(m, j, i)] : 0.0;
+      const double wv = w.u ? w.v[p2(m, j, i)] : 0.0;
       const long long p = p2(m, j, i);
       double S, D;
-      if (i < m.nx - 1) {
-        u_sd_x<CROSS, double>(m, kp, c, j, i, c.rt_u[p], U, V, S, D);
-        const double yv = S + D * x.u[p];
+      if (cr.hu(m)) {
+        cr.u_sd(m, kp, x.u, S, D);
+        const double yv = S + D * cr.U.c;
         y.u[p] = yv;
-        if (w.u) { acc[0] += w.u[p] * yv; acc[1] += yv * yv; }
+        acc[0] += wu * yv;
+        acc[1] += yv * yv;
       }
-      if (j < m.ny - 1) {
-        v_sd_x<CROSS, double>(m, kp, c, j, i, c.rt_v[p], U, V, S, D);
-        const double yv = S + D * x.v[p];
+      if (cr.hv(m)) {
+        cr.v_sd(m, kp, x.v, S, D);
+        const double yv = S + D * cr.V.c;
         y.v[p] = yv;
-        if (w.u) { acc[0] += w.v[p] * yv; acc[1] += yv * yv; }
+        acc[0] += wv * yv;
+        acc[1] += yv * yv;
       }
     }
   }
@@ -1930,29 +2020,35 @@ __global__ void __launch_bounds__(IMAU_WG) k_apply(const Member *__restrict__ me
 }
 
 // r = b - A x, rhat = r, p = v = 0; partials (r, r), (b, b)
+template <int CROSS>
 __global__ void __launch_bounds__(IMAU_WG) k_bicg_init(const Member *__restrict__ mem, const Tile *__restrict__ tiles,
                                                        const KP kp, const CoefP c, CVec2 x, Vec2 r, Vec2 rh, Vec2 pp,
                                                        Vec2 vv, const int *__restrict__ active,
                                                        double *__restrict__ partial) {
   TILE_SETUP
   double acc[2] = {0.0, 0.0};
-  const GAcc U{x.u, m}, V{x.v, m};
   if (j < m.ny && active[t.g]) {
-    FOR_TILE_ROWS {
+    FOR_TILE_ROWS_1 {
       const int i = t.i0 + ii;
       if (i >= m.nx) break;
+      CellRows<CROSS> cr;
+      cr.load(m, c, x.u, x.v, j, i);
+      const double tu = c.taudx[p2(m, j, i)];
+      const double tv = c.taudy[p2(m, j, i)];
       const long long p = p2(m, j, i);
-      double S, D, b;
-      if (i < m.nx - 1) {
-        u_row(m, kp, c, j, i, c.rt_u[p], U, V, S, D, b);
-        const double rv = b - (S + D * x.u[p]);
+      double S, D;
+      if (cr.hu(m)) {
+        cr.u_sd(m, kp, x.u, S, D);
+        const double b = u_rhs<CROSS>(m, c, j, i, cr.ru, tu, cr.k.nb0);
+        const double rv = b - (S + D * cr.U.c);
         r.u[p] = rv;
         if (rh.u) { rh.u[p] = rv; pp.u[p] = 0.0; vv.u[p] = 0.0; }
         acc[0] += rv * rv; acc[1] += b * b;
       }
-      if (j < m.ny - 1) {
-        v_row(m, kp, c, j, i, c.rt_v[p], U, V, S, D, b);
-        const double rv = b - (S + D * x.v[p]);
+      if (cr.hv(m)) {
+        cr.v_sd(m, kp, x.v, S, D);
+        const double b = v_rhs<CROSS>(m, c, j, i, cr.rv, tv, cr.k.nbw);
+        const double rv = b - (S + D * cr.V.c);
         r.v[p] = rv;
         if (rh.u) { rh.v[p] = rv; pp.v[p] = 0.0; vv.v[p] = 0.0; }
         acc[0] += rv * rv; acc[1] += b * b;
@@ -2244,7 +2340,8 @@ void apply(const Launch &L, const KP &kp, const Coef &c, const double *xu, const
 void bicg_init(const Launch &L, const KP &kp, const Coef &c, const double *xu, const double *xv, double *ru, double *rv,
                double *rhu, double *rhv, double *pu, double *pv, double *vu, double *vv, const int *active,
                double *partial) {
-  hipLaunchKernelGGL(k_bicg_init, dim3(L.ntiles), wg(), 0, L.s, L.mem, L.tiles, kp, to_p(c), CVec2{xu, xv}, Vec2{ru, rv},
+  auto k = kp.cross ? k_bicg_init<1> : k_bicg_init<0>;
+  hipLaunchKernelGGL(k, dim3(L.ntiles), wg(), 0, L.s, L.mem, L.tiles, kp, to_p(c), CVec2{xu, xv}, Vec2{ru, rv},
                      Vec2{rhu, rhv}, Vec2{pu, pv}, Vec2{vu, vv}, active, partial);
 }
 void bicg_p(const Launch &L, const double *ru, const double *rv, double *pu, double *pv, const double *vu,
@@ -2285,71 +2382,89 @@ void sor_color(const Launch &L, const KP &kp, const Coef &c, double *xu, double 
 // are kept orthonormal; scalars live on the device (sc[g*8 + ...]).
 // ---------------------------------------------------------------------------
 namespace gcr {
-enum { BETA = 0, INVN = IMAU_GCR_M, ALPHA = IMAU_GCR_M + 1, NV = 2 * IMAU_GCR_M + 2 };
+enum { BETA = 0, INVN = IMAU_GCR_M, ALPHA = IMAU_GCR_M + 1 };
 }
 
-// partial sums per tile: (q,Q_i) and (r,Q_i) for i < nj, (q,q), (r,q)
+// partial sums per tile: (q,Q_i) and (r,Q_i) for i < NJ, (q,q), (r,q); all of a
+// thread's values are loaded before the first product: 21.5 -> 8.4 us (first
+// step) and 11.0 (later ones) on 12 uneven ice caps of 96 to 512 a side,
+// 11.1 -> 5.3 and 6.4 on 8 of 256x256.
+template <int NJ>
 __global__ void __launch_bounds__(IMAU_WG) k_gcr_dots(const Member *__restrict__ mem, const Tile *__restrict__ tiles,
-                                                      CVec2 q, CVec2 r, GList Q, int nj,
-                                                      const int *__restrict__ active, double *__restrict__ partial) {
+                                                      CVec2 q, CVec2 r, GList Q, const int *__restrict__ active,
+                                                      double *__restrict__ partial) {
   TILE_SETUP
-  double acc[gcr::NV];
+  double acc[2 * NJ + 2];
 #pragma unroll
-  for (int k = 0; k < gcr::NV; ++k) acc[k] = 0.0;
+  for (int k = 0; k < 2 * NJ + 2; ++k) acc[k] = 0.0;
   if (j < m.ny && active[t.g]) {
-    FOR_TILE_ROWS {
-      const int i = t.i0 + ii;
-      if (i >= m.nx) break;
-      const long long p = p2(m, j, i);
-      for (int comp = 0; comp < 2; ++comp) {
-        if (comp == 0 ? (i >= m.nx - 1) : (j >= m.ny - 1)) continue;
-        const double qv = (comp == 0 ? q.u : q.v)[p], rv = (comp == 0 ? r.u : r.v)[p];
+    double qv[TROWS][2], rv[TROWS][2], w[TROWS][2][NJ ? NJ : 1];
+    bool ok[TROWS][2];
 #pragma unroll
-        for (int k = 0; k < IMAU_GCR_M; ++k)
-          if (k < nj) {
-            const double w = (comp == 0 ? Q.u[k] : Q.v[k])[p];
-            acc[k] += qv * w;
-            acc[IMAU_GCR_M + k] += rv * w;
-          }
-        acc[2 * IMAU_GCR_M] += qv * qv;
-        acc[2 * IMAU_GCR_M + 1] += rv * qv;
+    for (int a = 0; a < TROWS; ++a) {
+      const int i = t.i0 + (int)threadIdx.y + a * IMAU_WG_I;
+      const long long p = p2(m, j, min(i, m.nx - 1));
+      ok[a][0] = i < m.nx - 1;
+      ok[a][1] = i < m.nx && j < m.ny - 1;
+#pragma unroll
+      for (int comp = 0; comp < 2; ++comp) {
+        qv[a][comp] = (comp == 0 ? q.u : q.v)[p];
+        rv[a][comp] = (comp == 0 ? r.u : r.v)[p];
+#pragma unroll
+        for (int k = 0; k < NJ; ++k) w[a][comp][k] = (comp == 0 ? Q.u[k] : Q.v[k])[p];
       }
     }
+#pragma unroll
+    for (int a = 0; a < TROWS; ++a)
+#pragma unroll
+      for (int comp = 0; comp < 2; ++comp) {
+        if (!ok[a][comp]) continue;
+        const double x = qv[a][comp], y = rv[a][comp];
+#pragma unroll
+        for (int k = 0; k < NJ; ++k) {
+          acc[k] += x * w[a][comp][k];
+          acc[NJ + k] += y * w[a][comp][k];
+        }
+        acc[2 * NJ] += x * x;
+        acc[2 * NJ + 1] += y * x;
+      }
   }
-  block_sum_store<gcr::NV>(acc, partial + gcr::NV * (long long)tb);
+  block_sum_store<2 * NJ + 2>(acc, partial + (2 * NJ + 2) * (long long)tb);
 }
 
 // per member: beta_i = (q,Q_i), q' = q - sum beta_i Q_i, |q'| from the Gram
 // identity, alpha = (r, q'/|q'|)
+template <int NJ>
 __global__ void __launch_bounds__(256) k_gcr_scalar(const int *__restrict__ tstart, const double *__restrict__ partial,
-                                                    double *__restrict__ sc, const int *__restrict__ active, int nj) {
+                                                    double *__restrict__ sc, const int *__restrict__ active) {
+  constexpr int NV = 2 * NJ + 2;
   const int g = blockIdx.x;
   if (!active[g]) return;
   const int a = tstart[g], b = tstart[g + 1];
-  __shared__ double red[gcr::NV][256];
-  double s[gcr::NV];
+  __shared__ double red[NV][256];
+  double s[NV];
 #pragma unroll
-  for (int q = 0; q < gcr::NV; ++q) s[q] = 0.0;
+  for (int q = 0; q < NV; ++q) s[q] = 0.0;
   for (int k = a + (int)threadIdx.x; k < b; k += 256)
 #pragma unroll
-    for (int q = 0; q < gcr::NV; ++q) s[q] += partial[(long long)gcr::NV * k + q];
+    for (int q = 0; q < NV; ++q) s[q] += partial[(long long)NV * k + q];
 #pragma unroll
-  for (int q = 0; q < gcr::NV; ++q) red[q][threadIdx.x] = s[q];
+  for (int q = 0; q < NV; ++q) red[q][threadIdx.x] = s[q];
   __syncthreads();
   for (int w = 128; w > 0; w >>= 1) {
     if ((int)threadIdx.x < w)
 #pragma unroll
-      for (int q = 0; q < gcr::NV; ++q) red[q][threadIdx.x] += red[q][threadIdx.x + w];
+      for (int q = 0; q < NV; ++q) red[q][threadIdx.x] += red[q][threadIdx.x + w];
     __syncthreads();
   }
   if (threadIdx.x != 0) return;
   double *S = sc + g * bicg::NSC;
-  double qq = red[2 * IMAU_GCR_M][0], rq = red[2 * IMAU_GCR_M + 1][0];
-  for (int k = 0; k < IMAU_GCR_M; ++k) {
-    const double beta = (k < nj) ? red[k][0] : 0.0;
+  double qq = red[2 * NJ][0], rq = red[2 * NJ + 1][0];
+  for (int k = 0; k < NJ; ++k) {
+    const double beta = red[k][0];
     S[gcr::BETA + k] = beta;
     qq -= beta * beta;
-    rq -= beta * ((k < nj) ? red[IMAU_GCR_M + k][0] : 0.0);
+    rq -= beta * red[NJ + k][0];
   }
   const bool ok = qq > 0.0 && isfinite(qq);
   const double inv = ok ? 1.0 / sqrt(qq) : 0.0;
@@ -2357,10 +2472,12 @@ __global__ void __launch_bounds__(256) k_gcr_scalar(const int *__restrict__ tsta
   S[gcr::ALPHA] = ok ? rq * inv : 0.0;
 }
 
-// Q_nj = (q - sum beta_i Q_i)/|q'|, Z_nj likewise, x += alpha Z_nj, r -= alpha Q_nj;
-// q and z are read from, and replaced in, the slots Q_nj and Z_nj; partial (r,r)
+// Q_NJ = (q - sum beta_i Q_i)/|q'|, Z_NJ likewise, x += alpha Z_NJ, r -= alpha Q_NJ;
+// q and z are read from, and replaced in, the slots Q_NJ and Z_NJ; partial (r,r).
+// All of a thread's values are loaded before the first is used.
+template <int NJ>
 __global__ void __launch_bounds__(IMAU_WG) k_gcr_update(const Member *__restrict__ mem, const Tile *__restrict__ tiles,
-                                                        GList Q, GList Z, int nj, Vec2 x, Vec2 r,
+                                                        GList Q, GList Z, Vec2 x, Vec2 r,
                                                         const double *__restrict__ sc, const int *__restrict__ active,
                                                         double *__restrict__ partial) {
   TILE_SETUP
@@ -2368,34 +2485,51 @@ __global__ void __launch_bounds__(IMAU_WG) k_gcr_update(const Member *__restrict
   if (j < m.ny && active[t.g]) {
     const double *S = sc + t.g * bicg::NSC;
     const double inv = S[gcr::INVN], al = S[gcr::ALPHA];
-    double be[IMAU_GCR_M];
+    double be[NJ ? NJ : 1];
 #pragma unroll
-    for (int k = 0; k < IMAU_GCR_M; ++k) be[k] = S[gcr::BETA + k];
-    FOR_TILE_ROWS {
-      const int i = t.i0 + ii;
-      if (i >= m.nx) break;
-      const long long p = p2(m, j, i);
+    for (int k = 0; k < NJ; ++k) be[k] = S[gcr::BETA + k];
+    double qv[TROWS][2], zv[TROWS][2], xv[TROWS][2], rv[TROWS][2], wq[TROWS][2][NJ ? NJ : 1], wz[TROWS][2][NJ ? NJ : 1];
+    bool ok[TROWS][2];
+    long long p[TROWS];
+#pragma unroll
+    for (int a = 0; a < TROWS; ++a) {
+      const int i = t.i0 + (int)threadIdx.y + a * IMAU_WG_I;
+      p[a] = p2(m, j, min(i, m.nx - 1));
+      ok[a][0] = i < m.nx - 1;
+      ok[a][1] = i < m.nx && j < m.ny - 1;
+#pragma unroll
       for (int comp = 0; comp < 2; ++comp) {
-        if (comp == 0 ? (i >= m.nx - 1) : (j >= m.ny - 1)) continue;
-        double *qn = const_cast<double *>(comp == 0 ? Q.u[nj] : Q.v[nj]);
-        double *zn = const_cast<double *>(comp == 0 ? Z.u[nj] : Z.v[nj]);
-        double qv = qn[p], zv = zn[p];
+        qv[a][comp] = (comp == 0 ? Q.u[NJ] : Q.v[NJ])[p[a]];
+        zv[a][comp] = (comp == 0 ? Z.u[NJ] : Z.v[NJ])[p[a]];
+        xv[a][comp] = (comp == 0 ? x.u : x.v)[p[a]];
+        rv[a][comp] = (comp == 0 ? r.u : r.v)[p[a]];
 #pragma unroll
-        for (int k = 0; k < IMAU_GCR_M; ++k)
-          if (k < nj) {
-            qv -= be[k] * (comp == 0 ? Q.u[k] : Q.v[k])[p];
-            zv -= be[k] * (comp == 0 ? Z.u[k] : Z.v[k])[p];
-          }
-        qv *= inv;
-        zv *= inv;
-        qn[p] = qv;
-        zn[p] = zv;
-        (comp == 0 ? x.u : x.v)[p] += al * zv;
-        double &rr = (comp == 0 ? r.u : r.v)[p];
-        rr -= al * qv;
-        acc[0] += rr * rr;
+        for (int k = 0; k < NJ; ++k) {
+          wq[a][comp][k] = (comp == 0 ? Q.u[k] : Q.v[k])[p[a]];
+          wz[a][comp][k] = (comp == 0 ? Z.u[k] : Z.v[k])[p[a]];
+        }
       }
     }
+#pragma unroll
+    for (int a = 0; a < TROWS; ++a)
+#pragma unroll
+      for (int comp = 0; comp < 2; ++comp) {
+        if (!ok[a][comp]) continue;
+        double q = qv[a][comp], z = zv[a][comp];
+#pragma unroll
+        for (int k = 0; k < NJ; ++k) {
+          q -= be[k] * wq[a][comp][k];
+          z -= be[k] * wz[a][comp][k];
+        }
+        q *= inv;
+        z *= inv;
+        const_cast<double *>(comp == 0 ? Q.u[NJ] : Q.v[NJ])[p[a]] = q;
+        const_cast<double *>(comp == 0 ? Z.u[NJ] : Z.v[NJ])[p[a]] = z;
+        (comp == 0 ? x.u : x.v)[p[a]] = xv[a][comp] + al * z;
+        const double rn = rv[a][comp] - al * q;
+        (comp == 0 ? r.u : r.v)[p[a]] = rn;
+        acc[0] += rn * rn;
+      }
   }
   block_sum_store<2>(acc, partial + 2 * (long long)tb);
 }
@@ -2403,17 +2537,20 @@ __global__ void __launch_bounds__(IMAU_WG) k_gcr_update(const Member *__restrict
 namespace imau {
 void gcr_dots(const Launch &L, const double *qu, const double *qv, const double *ru, const double *rv, const GList &Q,
               int nj, const int *active, double *partial) {
-  hipLaunchKernelGGL(k_gcr_dots, dim3(L.ntiles), wg(), 0, L.s, L.mem, L.tiles, CVec2{qu, qv}, CVec2{ru, rv}, Q, nj,
-                     active, partial);
+  static_assert(IMAU_GCR_M == 4, "one specialisation per number of stored directions");
+  auto k = nj == 0 ? k_gcr_dots<0> : nj == 1 ? k_gcr_dots<1> : nj == 2 ? k_gcr_dots<2> : k_gcr_dots<3>;
+  hipLaunchKernelGGL(k, dim3(L.ntiles), wg(), 0, L.s, L.mem, L.tiles, CVec2{qu, qv}, CVec2{ru, rv}, Q, active, partial);
 }
 void gcr_scalar(hipStream_t s, int ngrids, const int *tstart, const double *partial, double *sc, const int *active,
                 int nj) {
-  hipLaunchKernelGGL(k_gcr_scalar, dim3(ngrids), dim3(256), 0, s, tstart, partial, sc, active, nj);
+  auto k = nj == 0 ? k_gcr_scalar<0> : nj == 1 ? k_gcr_scalar<1> : nj == 2 ? k_gcr_scalar<2> : k_gcr_scalar<3>;
+  hipLaunchKernelGGL(k, dim3(ngrids), dim3(256), 0, s, tstart, partial, sc, active);
 }
 void gcr_update(const Launch &L, const GList &Q, const GList &Z, int nj, double *xu, double *xv, double *ru, double *rv,
                 const double *sc, const int *active, double *partial) {
-  hipLaunchKernelGGL(k_gcr_update, dim3(L.ntiles), wg(), 0, L.s, L.mem, L.tiles, Q, Z, nj, Vec2{xu, xv},
-                     Vec2{ru, rv}, sc, active, partial);
+  auto k = nj == 0 ? k_gcr_update<0> : nj == 1 ? k_gcr_update<1> : nj == 2 ? k_gcr_update<2> : k_gcr_update<3>;
+  hipLaunchKernelGGL(k, dim3(L.ntiles), wg(), 0, L.s, L.mem, L.tiles, Q, Z, Vec2{xu, xv}, Vec2{ru, rv}, sc, active,
+                     partial);
 }
 }  // namespace imau
 
