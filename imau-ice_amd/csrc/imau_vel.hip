@@ -2647,7 +2647,7 @@ void net_plan_build(const Pool &pool, hipStream_t s, imau_net_plan *N, int nimg,
       if (l == 0) off0[g] = off;
       off += (long long)r * c;
       for (int r0 = 0; r0 < r; r0 += IMAU_NET_TR)
-        for (int c0 = 0; c0 < c; c0 += IMAU_NET_TC) tl.push_back(imau::net::NTile{g, r0, c0, 0});
+        for (int c0 = 0; c0 < c; c0 += IMAU_NET_TC) tl.push_back(imau::net::NTile{g, r0, c0, r, c, 0, im[g].off});
     }
     N->npix[l] = off;
     N->ntiles[l] = (int)tl.size();

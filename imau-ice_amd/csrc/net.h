@@ -25,8 +25,9 @@ struct NImg {
   int rows, cols;
   long long off;
 };
-struct NTile {
-  int img, r0, c0, pad;
+struct NTile {  // with its image's extents and offset, so that a kernel needs one look-up
+  int img, r0, c0, rows, cols, pad;
+  long long off;
 };
 struct LevelView {
   const NImg *img;

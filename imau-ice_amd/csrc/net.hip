@@ -1,13 +1,13 @@
 // net.hip -- kernels of the warm-start network: 3x3 convolutions on the
-// matrix cores (v_mfma_f32_16x16x32_bf16 for 32 input channels,
-// v_mfma_f32_16x16x16_bf16 for 16: BF16 operands, FP32 accumulation),
-// their weight gradients, 2x2 pooling, upsampling with skip addition, the
+// matrix cores (v_mfma_f32_16x16x32_bf16 for 32 input channels and for the
+// weight gradients, v_mfma_f32_16x16x16_bf16 for 16: BF16 operands, FP32
+// accumulation), 2x2 pooling, upsampling with skip addition, the
 // backward passes of those, a weighted squared-error loss and Adam.
 //
 // Convolution as a matrix product per tile: D[cout][pixel] = W[cout][9 cin] X[9 cin][pixel],
 // one wavefront per tile of IMAU_NET_TR x IMAU_NET_TC pixels (IMAU_NET_TR
 // column blocks of 16 pixels), the layer's weights held in registers as the A
-// operands, the input pixels (channels contiguous) loaded straight from HBM as
+// operands, the input pixels (channels contiguous) staged in LDS as
 // the B operands.  Operand layout of the 16x16x16 instruction, lane l:
 // A[i][k] with i = l % 16, k = 4 (l / 16) + e;  B[k][j] with j = l % 16,
 // k = 4 (l / 16) + e;  D[i][j] with j = l % 16, i = 4 (l / 16) + e  (e = 0..3).
@@ -40,288 +40,307 @@ __device__ __forceinline__ void st4(uint16_t *p, s4 v) { *reinterpret_cast<s4 *>
 // ---------------------------------------------------------------------------
 // convolution
 // ---------------------------------------------------------------------------
+typedef __bf16 b8 __attribute__((ext_vector_type(8)));
+typedef float f2 __attribute__((ext_vector_type(2)));
+typedef float f8 __attribute__((ext_vector_type(8)));
+// 16-byte accesses to global memory need no more than a dword's alignment
+typedef b8 b8u __attribute__((aligned(4)));
+typedef f2 f2u __attribute__((aligned(4)));
+__device__ __forceinline__ b8 ld8(const uint16_t *p) { return *reinterpret_cast<const b8u *>(p); }
+
+// LDS written and read by the same wavefront: its LDS operations complete in
+// order, so only the compiler has to keep them so
+__device__ __forceinline__ void wave_lds_sync() {
+  __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
+  __builtin_amdgcn_wave_barrier();
+  __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
+}
+
+// Bound by its bytes: CIN + COUT channels per pixel.  Each wavefront stages its
+// tile plus a one-pixel halo ((TR+2) x (TC+2) pixels) in LDS with 16-byte loads
+// that are all in flight together (the tile's descriptor came a tile earlier;
+// outside the image they read pixel (0, 0)
+// and are replaced by zeros); the next tile's loads are issued before this
+// one's products.  A staged row serves the three tile rows that it touches, in
+// the order of the taps.  32 channels: one v_mfma_f32_16x16x32_bf16 per tap and
+// 16 outputs (lane l holds k = 8 (l / 16) + e of its row / column), pixels
+// padded to 40 channels against bank conflicts; 16 channels:
+// v_mfma_f32_16x16x16_bf16.  With 32 outputs the weight rows are dealt so that
+// a lane ends with 8 neighbouring channels, one 16-byte store per pixel.  The
+// tiles are dealt to the 8 XCDs in contiguous runs, so halos are found in
+// their L2.  Over 1.37 million pixels (floors at the rate of a
+// copy: 36 us for 32 -> 32, 27 for 16 -> 32, 20 for 32 -> 2): 32 -> 32 73 -> 38
+// us, 16 -> 32 95 -> 32 (it staged nothing), 32 -> 2 FP32 33 -> 24.
 template <int CIN, int COUT, bool OUTF>
-__global__ void __launch_bounds__(256) k_conv(const NImg *__restrict__ img, const NTile *__restrict__ tiles,
-                                              int ntiles, const uint16_t *__restrict__ x,
+__global__ void __launch_bounds__(256) k_conv(const NTile *__restrict__ tiles, int ntiles,
+                                              const uint16_t *__restrict__ x,
                                               const uint16_t *__restrict__ w, const float *__restrict__ bias,
                                               int relu, void *__restrict__ yv) {
-  constexpr int NCH = CIN / 16, NCT = COUT / 16;
-  const int lane = threadIdx.x & 63, lc = lane & 15, lk = lane >> 4;
-  const int wid = blockIdx.x * 4 + (threadIdx.x >> 6);
-  if (wid >= ntiles) return;  // uniform per wavefront
-  s4 wa[9][NCH][NCT];
+  constexpr int NCT = COUT / 16, KL = CIN / 4;  // KL: channels per lane and instruction
+  constexpr int XR = TR + 2, XC = TC + 2, CP = CIN == 32 ? 40 : 16, WSZ = XR * XC * CP;
+  constexpr int CH = CIN / 8, NQ = XR * XC * CH, NL = (NQ + 63) / 64;  // 16-byte pieces of a pixel, of a tile, per lane
+  typedef short sk __attribute__((ext_vector_type(KL)));
+  __shared__ __align__(16) uint16_t sx[4 * WSZ];
+  const int lane = threadIdx.x & 63, lc = lane & 15, lk = lane >> 4, wv = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+  uint16_t *my = sx + wv * WSZ;
+  // blocks b, b + 8, .. run on one XCD
+  const int ng = (ntiles + 3) / 4, gx = (ng + 7) / 8, gs = (int)gridDim.x / 8;
+  const int g0 = ((int)blockIdx.x & 7) * gx, g1 = min(ng, g0 + gx);
+  int tix = 4 * (g0 + ((int)blockIdx.x >> 3)) + wv;
+  const int tend = min(ntiles, 4 * g1);
+  if (tix >= tend) return;  // uniform per wavefront; there is no barrier below
+
+  // output channel of row i of weight block ct
+  auto co_of = [](int ct, int i) { return NCT == 2 ? 8 * (i >> 2) + 4 * ct + (i & 3) : i; };
+  b8 pre[NL];
+  auto load = [&](const NTile &t) {
+    const uint16_t *xi = x + t.off * CIN;
+#pragma unroll
+    for (int l = 0; l < NL; ++l) {
+      const int q = lane + 64 * l, px = q / CH, ch = q % CH;
+      const int hr = px / XC, hc = px - hr * XC;
+      const int rr = t.r0 + hr - 1, cc = t.c0 + hc - 1;
+      const bool ok = rr >= 0 && rr < t.rows && cc >= 0 && cc < t.cols;
+      const b8 v = ld8(xi + (ok ? ((long long)rr * t.cols + cc) * CIN : 0) + 8 * ch);
+      pre[l] = ok ? v : b8{};
+    }
+  };
+  const int dt = 4 * gs;
+  NTile tc = tiles[tix], tn = tiles[min(tix + dt, ntiles - 1)];
+  load(tc);
+  sk wa[9][NCT];
 #pragma unroll
   for (int tap = 0; tap < 9; ++tap)
 #pragma unroll
-    for (int ch = 0; ch < NCH; ++ch)
-#pragma unroll
-      for (int ct = 0; ct < NCT; ++ct)
-        wa[tap][ch][ct] = ld4(w + ((size_t)(tap * COUT + ct * 16 + lc) * CIN + ch * 16 + 4 * lk));
+    for (int ct = 0; ct < NCT; ++ct)
+      wa[tap][ct] = *reinterpret_cast<const sk *>(w + (size_t)(tap * COUT + co_of(ct, lc)) * CIN + KL * lk);
   float bs[NCT][4];
 #pragma unroll
   for (int ct = 0; ct < NCT; ++ct)
 #pragma unroll
-    for (int e = 0; e < 4; ++e) bs[ct][e] = bias ? bias[ct * 16 + 4 * lk + e] : 0.0f;
+    for (int e = 0; e < 4; ++e) bs[ct][e] = bias ? bias[co_of(ct, 4 * lk + e)] : 0.0f;
 
-  for (int tix = wid; tix < ntiles; tix += gridDim.x * 4) {
-    const NTile t = tiles[tix];
-    const NImg im = img[t.img];
+  for (;;) {
+#pragma unroll
+    for (int l = 0; l < NL; ++l) {
+      const int q = lane + 64 * l;
+      if (64 * l + 63 < NQ || q < NQ) *reinterpret_cast<b8 *>(my + (q / CH) * CP + 8 * (q % CH)) = pre[l];
+    }
+    wave_lds_sync();
+    tix += dt;
+    const bool more = tix < tend;
+    const NTile tl = tn;
+    if (more) {
+      load(tl);
+      tn = tiles[min(tix + dt, ntiles - 1)];
+    }
     f4 acc[TR][NCT];
 #pragma unroll
     for (int r = 0; r < TR; ++r)
 #pragma unroll
       for (int ct = 0; ct < NCT; ++ct) acc[r][ct] = f4{0.0f, 0.0f, 0.0f, 0.0f};
 #pragma unroll
-    for (int tap = 0; tap < 9; ++tap) {
-      const int dr = tap / 3 - 1, dc = tap % 3 - 1;
-      const int c = t.c0 + lc + dc;
-      const bool cok = c >= 0 && c < im.cols;
+    for (int hr = 0; hr < XR; ++hr)
 #pragma unroll
-      for (int r = 0; r < TR; ++r) {
-        const int rr = t.r0 + r + dr;
-        const bool ok = cok && rr >= 0 && rr < im.rows;
-        const uint16_t *px = x + (im.off + (long long)rr * im.cols + c) * CIN + 4 * lk;
+      for (int dc = 0; dc < 3; ++dc) {
+        const sk b = *reinterpret_cast<const sk *>(my + (hr * XC + lc + dc) * CP + KL * lk);
 #pragma unroll
-        for (int ch = 0; ch < NCH; ++ch) {
-          s4 b = s4{0, 0, 0, 0};
-          if (ok) b = ld4(px + ch * 16);
+        for (int dr = 0; dr < 3; ++dr) {
+          const int r = hr - dr;
+          if (r < 0 || r >= TR) continue;
 #pragma unroll
-          for (int ct = 0; ct < NCT; ++ct)
-            acc[r][ct] = __builtin_amdgcn_mfma_f32_16x16x16bf16_1k(wa[tap][ch][ct], b, acc[r][ct], 0, 0, 0);
+          for (int ct = 0; ct < NCT; ++ct) {
+            if constexpr (CIN == 32)
+              acc[r][ct] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(
+                  __builtin_bit_cast(b8, wa[3 * dr + dc][ct]), __builtin_bit_cast(b8, b), acc[r][ct], 0, 0, 0);
+            else
+              acc[r][ct] = __builtin_amdgcn_mfma_f32_16x16x16bf16_1k(wa[3 * dr + dc][ct], b, acc[r][ct], 0, 0, 0);
+          }
         }
       }
-    }
-    const int c = t.c0 + lc;
+    const int c = tc.c0 + lc;
 #pragma unroll
     for (int r = 0; r < TR; ++r) {
-      const int rr = t.r0 + r;
-      if (rr >= im.rows || c >= im.cols) continue;
-      const long long pix = im.off + (long long)rr * im.cols + c;
+      const int rr = tc.r0 + r;
+      float v[NCT * 4];
 #pragma unroll
-      for (int ct = 0; ct < NCT; ++ct) {
-        float v[4];
+      for (int ct = 0; ct < NCT; ++ct)
 #pragma unroll
         for (int e = 0; e < 4; ++e) {
-          v[e] = acc[r][ct][e] + bs[ct][e];
-          if (relu) v[e] = fmaxf(v[e], 0.0f);
+          const float s = acc[r][ct][e] + bs[ct][e];
+          v[4 * ct + e] = relu ? fmaxf(s, 0.0f) : s;
         }
-        if constexpr (OUTF) {
-          if (ct == 0 && lk == 0) {
-            float *y = static_cast<float *>(yv);
-            y[2 * pix] = v[0];
-            y[2 * pix + 1] = v[1];
-          }
+      if (rr >= tc.rows || c >= tc.cols) continue;
+      const long long pix = tc.off + (long long)rr * tc.cols + c;
+      if constexpr (OUTF) {
+        if (lk == 0) *reinterpret_cast<f2u *>(static_cast<float *>(yv) + 2 * pix) = f2{v[0], v[1]};
+      } else {
+        uint16_t *yp = static_cast<uint16_t *>(yv) + pix * COUT + NCT * 4 * lk;
+        if constexpr (NCT == 2) {
+          const f8 o = {v[0], v[1], v[2], v[3], v[4], v[5], v[6], v[7]};
+          *reinterpret_cast<b8u *>(yp) = __builtin_convertvector(o, b8);
         } else {
-          s4 o;
-#pragma unroll
-          for (int e = 0; e < 4; ++e) o[e] = (short)f2bf(v[e]);
-          st4(static_cast<uint16_t *>(yv) + pix * COUT + ct * 16 + 4 * lk, o);
+          typedef __bf16 b4 __attribute__((ext_vector_type(4)));
+          const f4 o = {v[0], v[1], v[2], v[3]};
+          *reinterpret_cast<b4 *>(yp) = __builtin_convertvector(o, b4);
         }
       }
     }
+    if (!more) break;
+    tc = tl;
+    wave_lds_sync();
   }
 }
 
-// The same convolution for 32 input channels on v_mfma_f32_16x16x32_bf16: one
-// instruction takes all 32 channels of a tap (lane l holds k = 8 (l / 16) + e,
-// e = 0..7, of its row / column), with 16-byte operand loads.
-typedef __bf16 b8 __attribute__((ext_vector_type(8)));
-__device__ __forceinline__ b8 ld8(const uint16_t *p) { return *reinterpret_cast<const b8 *>(p); }
+// Weight and bias gradients: dw[tap][co][ci] = G^T[co][pixels] X_tap[pixels][ci].
+// A workgroup of four wavefronts sums its tiles in registers and writes one
+// partial; sum_partials adds them in a fixed order.  Each wavefront owns one 16
+// x 16 block of (co, ci) for all nine taps (36 sums per lane, and with two such
+// blocks only, every second pair of tile rows), so that 4 workgroups fit on a
+// CU.  The tile's gradient (64 pixels) and input with a one-pixel halo are
+// staged in LDS transposed, [channel][pixel], two neighbouring pixels per write
+// (lanes of neighbouring pixels swap half their channels), so that a lane's 8
+// pixels of an operand are one 16-byte read, and the three column taps come
+// from the same 10 pixels, shifted.  Two rows of a tile (32 pixels) make one
+// v_mfma_f32_16x16x32_bf16.  The channel pitches (76 and 36 dwords) put the 16
+// channels of a read on distinct banks.  The next tile's loads are issued
+// before this one's products; two buffers, one barrier per tile.  The bias
+// gradient is a product with ones.  Over 16 images of 256 x 256 (floor 28 us):
+// 32 -> 32 channels 95 -> 58 us against one wavefront per workgroup with all
+// blocks' sums in 144 registers and 2-byte LDS reads, 16 -> 32 69 -> 38, 32 -> 16
+// 71 -> 42.  512 and 768 workgroups instead of at most 1024: 69 and 60 us, 1280: 69.
+constexpr int GP = TR * TC + 8;                   // pitch of a channel of g
+constexpr int XW = 24, XP = (TR + 2) * XW + 8;    // pitch of a row and of a channel of x
 
-template <int COUT, bool OUTF>
-__global__ void __launch_bounds__(256) k_conv32(const NImg *__restrict__ img, const NTile *__restrict__ tiles,
-                                                int ntiles, const uint16_t *__restrict__ x,
-                                                const uint16_t *__restrict__ w, const float *__restrict__ bias,
-                                                int relu, void *__restrict__ yv) {
-  constexpr int CIN = 32, NCT = COUT / 16;
-  // each wavefront stages its tile plus a one-pixel halo ((TR+2) x (TC+2)
-  // pixels, 32 channels, rows padded to 40 channels against bank conflicts)
-  // in LDS once, instead of nine overlapping global loads per tap
-  constexpr int XR = TR + 2, XC = TC + 2, CP = 40, WSZ = XR * XC * CP;
-  __shared__ __align__(16) uint16_t sx[4 * WSZ];
-  const int lane = threadIdx.x & 63, lc = lane & 15, lk = lane >> 4, wv = threadIdx.x >> 6;
-  uint16_t *my = sx + wv * WSZ;
-  b8 wa[9][NCT];
-#pragma unroll
-  for (int tap = 0; tap < 9; ++tap)
-#pragma unroll
-    for (int ct = 0; ct < NCT; ++ct) wa[tap][ct] = ld8(w + ((size_t)(tap * COUT + ct * 16 + lc) * CIN + 8 * lk));
-  float bs[NCT][4];
-#pragma unroll
-  for (int ct = 0; ct < NCT; ++ct)
-#pragma unroll
-    for (int e = 0; e < 4; ++e) bs[ct][e] = bias ? bias[ct * 16 + 4 * lk + e] : 0.0f;
-
-  // the same number of rounds for every wavefront of the block (barriers)
-  for (int base = blockIdx.x * 4; base < ntiles; base += gridDim.x * 4) {
-    const int tix = base + wv;
-    const bool have = tix < ntiles;
-    NTile t = NTile{0, 0, 0, 0};
-    NImg im = NImg{0, 0, 0};
-    if (have) {
-      t = tiles[tix];
-      im = img[t.img];
-    }
-    if (have)
-      for (int q = lane; q < XR * XC * 4; q += 64) {
-        const int px = q >> 2, ch = q & 3;
-        const int hr = px / XC, hc = px - hr * XC;
-        const int rr = t.r0 + hr - 1, cc = t.c0 + hc - 1;
-        b8 v = {};
-        if (rr >= 0 && rr < im.rows && cc >= 0 && cc < im.cols)
-          v = ld8(x + (im.off + (long long)rr * im.cols + cc) * CIN + 8 * ch);
-        *reinterpret_cast<b8 *>(my + px * CP + 8 * ch) = v;
-      }
-    __syncthreads();
-    if (have) {
-      f4 acc[TR][NCT];
-#pragma unroll
-      for (int r = 0; r < TR; ++r)
-#pragma unroll
-        for (int ct = 0; ct < NCT; ++ct) acc[r][ct] = f4{0.0f, 0.0f, 0.0f, 0.0f};
-#pragma unroll
-      for (int tap = 0; tap < 9; ++tap) {
-        const int dr = tap / 3 - 1, dc = tap % 3 - 1;
-#pragma unroll
-        for (int r = 0; r < TR; ++r) {
-          const b8 b = *reinterpret_cast<const b8 *>(my + ((r + 1 + dr) * XC + lc + 1 + dc) * CP + 8 * lk);
-#pragma unroll
-          for (int ct = 0; ct < NCT; ++ct)
-            acc[r][ct] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(wa[tap][ct], b, acc[r][ct], 0, 0, 0);
-        }
-      }
-      const int c = t.c0 + lc;
-#pragma unroll
-      for (int r = 0; r < TR; ++r) {
-        const int rr = t.r0 + r;
-        if (rr >= im.rows || c >= im.cols) continue;
-        const long long pix = im.off + (long long)rr * im.cols + c;
-#pragma unroll
-        for (int ct = 0; ct < NCT; ++ct) {
-          float v[4];
-#pragma unroll
-          for (int e = 0; e < 4; ++e) {
-            v[e] = acc[r][ct][e] + bs[ct][e];
-            if (relu) v[e] = fmaxf(v[e], 0.0f);
-          }
-          if constexpr (OUTF) {
-            if (ct == 0 && lk == 0) {
-              float *y = static_cast<float *>(yv);
-              y[2 * pix] = v[0];
-              y[2 * pix + 1] = v[1];
-            }
-          } else {
-            s4 o;
-#pragma unroll
-            for (int e = 0; e < 4; ++e) o[e] = (short)f2bf(v[e]);
-            st4(static_cast<uint16_t *>(yv) + pix * COUT + ct * 16 + 4 * lk, o);
-          }
-        }
-      }
-    }
-    __syncthreads();
-  }
-}
-
-// weight and bias gradients: per tile, the gradient g (64 pixels x COUT) and
-// the input x with a one-pixel halo ((TR+2) x (TC+2) pixels x CIN) are staged in
-// LDS; for each tap D[co][ci] += G^T[co][pixels] X_tap[pixels][ci] with K = 16
-// pixels (one tile row) per instruction.  Each workgroup (one wavefront) sums
-// its tiles in registers and writes one partial; sum_partials adds them in a
-// fixed order.
 template <int CIN, int COUT>
-__global__ void __launch_bounds__(64) k_conv_dw(const NImg *__restrict__ img, const NTile *__restrict__ tiles,
-                                                int ntiles, const uint16_t *__restrict__ g,
-                                                const uint16_t *__restrict__ x, float *__restrict__ part) {
-  constexpr int NCI = CIN / 16, NCO = COUT / 16;
-  constexpr int XR = TR + 2, XC = TC + 2;
-  constexpr int GP = COUT + 2, XP = CIN + 2;  // padded rows (LDS banks)
-  __shared__ uint16_t sg[TR * TC * GP];
-  __shared__ uint16_t sx[XR * XC * XP];
-  const int lane = threadIdx.x, lc = lane & 15, lk = lane >> 4;
-  f4 acc[9][NCO][NCI];
+__global__ void __launch_bounds__(256) k_conv_dw(const NTile *__restrict__ tiles, int ntiles,
+                                                 const uint16_t *__restrict__ g,
+                                                 const uint16_t *__restrict__ x, float *__restrict__ part) {
+  typedef uint32_t u4 __attribute__((ext_vector_type(4)));
+  constexpr int NCI = CIN / 16, NCO = COUT / 16, NB = NCI * NCO, WB = 4 / NB;  // WB: wavefronts per (co, ci) block
+  static_assert(TR == 4 && TC == 16 && (NB == 2 || NB == 4), "");
+  constexpr int XC = TC + 2, GH = COUT / 8, XH = CIN / 8;
+  constexpr int NG = TR * TC * GH, NX = (TR + 2) * XC * XH, LX = (NX + 255) / 256;
+  constexpr int BUF = COUT * GP + CIN * XP, RED = WB == 2 ? 2 * 10 * 64 * 8 : 0;  // uint16
+  __shared__ __align__(16) uint16_t sm[2 * BUF > RED ? 2 * BUF : RED];
+  const int tid = threadIdx.x, lane = tid & 63, lc = lane & 15, lk = lane >> 4, wv = tid >> 6;
+  const int co = wv % NCO, ci = (wv / NCO) % NCI, wr = wv / NB;
+  f4 acc[9], accb = f4{0.0f, 0.0f, 0.0f, 0.0f};
 #pragma unroll
-  for (int tap = 0; tap < 9; ++tap)
+  for (int tap = 0; tap < 9; ++tap) acc[tap] = f4{0.0f, 0.0f, 0.0f, 0.0f};
+  const short one = 0x3f80;
+  typedef short s8 __attribute__((ext_vector_type(8)));
+  const b8 ones = __builtin_bit_cast(b8, s8{one, one, one, one, one, one, one, one});
+
+  u4 pg, pxr[LX];
+  auto load = [&](const NTile &t) {
+    const u4 z = {0, 0, 0, 0};
+    if (NG == 256 || tid < NG) {
+      const int px = tid / GH, ch = tid % GH;
+      const int rr = t.r0 + px / TC, cc = t.c0 + px % TC;
+      const bool ok = rr < t.rows && cc < t.cols;
+      const b8 v = ld8(g + (t.off + (ok ? (long long)rr * t.cols + cc : 0)) * COUT + 8 * ch);
+      pg = ok ? __builtin_bit_cast(u4, v) : z;
+    } else {
+      pg = z;
+    }
 #pragma unroll
-    for (int a = 0; a < NCO; ++a)
-#pragma unroll
-      for (int b = 0; b < NCI; ++b) acc[tap][a][b] = f4{0.0f, 0.0f, 0.0f, 0.0f};
-  float bacc = 0.0f;
-  for (int tix = blockIdx.x; tix < ntiles; tix += gridDim.x) {
-    const NTile t = tiles[tix];
-    const NImg im = img[t.img];
+    for (int l = 0; l < LX; ++l) {
+      const int q = tid + 256 * l, px = q / XH, ch = q % XH;
+      const int rr = t.r0 + px / XC - 1, cc = t.c0 + px % XC - 1;
+      const bool ok = q < NX && rr >= 0 && rr < t.rows && cc >= 0 && cc < t.cols;
+      const b8 v = ld8(x + (t.off + (ok ? (long long)rr * t.cols + cc : 0)) * CIN + 8 * ch);
+      pxr[l] = ok ? __builtin_bit_cast(u4, v) : z;
+    }
+  };
+  // 8 channels of pixel p (this lane) and of its neighbour p ^ 1 (lane ^ H) to
+  // 4 channels of both: four dwords at d, d + pitch, ..
+  auto put = [&](u4 v, int H, uint16_t *d, int pitch, bool odd, bool ok) {
+    const uint32_t r0 = __shfl_xor(odd ? v[0] : v[2], H), r1 = __shfl_xor(odd ? v[1] : v[3], H);
+    if (!ok) return;
+    const uint32_t a0 = odd ? r0 : v[0], b0 = odd ? v[2] : r0, a1 = odd ? r1 : v[1], b1 = odd ? v[3] : r1;
+    uint32_t *o = reinterpret_cast<uint32_t *>(d);
+    o[0] = (a0 & 0xffffu) | (b0 << 16);
+    o[pitch / 2] = (a0 >> 16) | (b0 & 0xffff0000u);
+    o[pitch] = (a1 & 0xffffu) | (b1 << 16);
+    o[3 * (pitch / 2)] = (a1 >> 16) | (b1 & 0xffff0000u);
+  };
+
+  // blocks b, b + 8, .. run on one XCD: each XCD takes a contiguous run of tiles
+  const int nb = (int)gridDim.x, runs = nb % 8 == 0 ? 8 : 1, gx = (ntiles + runs - 1) / runs;
+  int tix = ((int)blockIdx.x % runs) * gx + (int)blockIdx.x / runs;
+  const int tend = min(ntiles, ((int)blockIdx.x % runs + 1) * gx);
+  const int dt = nb / runs;
+  NTile tn = tiles[min(tix + dt, ntiles - 1)];
+  if (tix < tend) load(tiles[tix]);
+  for (int k = 0; tix < tend; k ^= 1) {
+    uint16_t *sg = sm + k * BUF, *sx = sg + COUT * GP;
     {
-      const int rr = t.r0 + (lane >> 4), cc = t.c0 + (lane & 15);
-      const bool ok = rr < im.rows && cc < im.cols;
-      const uint16_t *src = g + (im.off + (long long)rr * im.cols + cc) * COUT;
-#pragma unroll
-      for (int k = 0; k < COUT; k += 4) {
-        s4 v = s4{0, 0, 0, 0};
-        if (ok) v = ld4(src + k);
-#pragma unroll
-        for (int e = 0; e < 4; ++e) sg[lane * GP + k + e] = (uint16_t)v[e];
-      }
+      const int px = tid / GH, ch = tid % GH, odd = px & 1;
+      put(pg, GH, sg + (8 * ch + 4 * odd) * GP + (px & ~1), GP, odd, NG == 256 || tid < NG);
     }
-    for (int q = lane; q < XR * XC; q += 64) {
-      const int hr = q / XC, hc = q - hr * XC;
-      const int rr = t.r0 + hr - 1, cc = t.c0 + hc - 1;
-      const bool ok = rr >= 0 && rr < im.rows && cc >= 0 && cc < im.cols;
-      const uint16_t *src = x + (im.off + (long long)rr * im.cols + cc) * CIN;
 #pragma unroll
-      for (int k = 0; k < CIN; k += 4) {
-        s4 v = s4{0, 0, 0, 0};
-        if (ok) v = ld4(src + k);
-#pragma unroll
-        for (int e = 0; e < 4; ++e) sx[q * XP + k + e] = (uint16_t)v[e];
-      }
+    for (int l = 0; l < LX; ++l) {
+      const int q = tid + 256 * l, px = q / XH, ch = q % XH, odd = px & 1;
+      put(pxr[l], XH, sx + (8 * ch + 4 * odd) * XP + px / XC * XW + (px % XC & ~1), XP, odd, q < NX);
     }
     __syncthreads();
-    if (lane < COUT)
-      for (int p = 0; p < TR * TC; ++p) bacc += bf2f(sg[p * GP + lane]);
+    tix += dt;
+    if (tix < tend) {
+      load(tn);
+      tn = tiles[min(tix + dt, ntiles - 1)];
+    }
 #pragma unroll
-    for (int tap = 0; tap < 9; ++tap) {
-      const int dr = tap / 3 - 1, dc = tap % 3 - 1;
+    for (int rp = 0; rp < TR / 2; ++rp) {
+      if (WB == 2 && rp != wr) continue;
+      const b8 a = *reinterpret_cast<const b8 *>(sg + (co * 16 + lc) * GP + 32 * rp + 8 * lk);
+      if (ci == 0) accb = __builtin_amdgcn_mfma_f32_16x16x32_bf16(a, ones, accb, 0, 0, 0);
 #pragma unroll
-      for (int r = 0; r < TR; ++r) {
-        s4 a[NCO], b[NCI];
-#pragma unroll
-        for (int co = 0; co < NCO; ++co)
-#pragma unroll
-          for (int e = 0; e < 4; ++e) a[co][e] = (short)sg[(r * TC + 4 * lk + e) * GP + co * 16 + lc];
-#pragma unroll
-        for (int ci = 0; ci < NCI; ++ci)
-#pragma unroll
-          for (int e = 0; e < 4; ++e)
-            b[ci][e] = (short)sx[((r + 1 + dr) * XC + 4 * lk + e + 1 + dc) * XP + ci * 16 + lc];
-#pragma unroll
-        for (int co = 0; co < NCO; ++co)
-#pragma unroll
-          for (int ci = 0; ci < NCI; ++ci)
-            acc[tap][co][ci] = __builtin_amdgcn_mfma_f32_16x16x16bf16_1k(a[co], b[ci], acc[tap][co][ci], 0, 0, 0);
+      for (int dr = 0; dr < 3; ++dr) {
+        const uint16_t *p = sx + (ci * 16 + lc) * XP + (2 * rp + (lk >> 1) + dr) * XW + 8 * (lk & 1);
+        const u4 w = *reinterpret_cast<const u4 *>(p);
+        const uint32_t w4 = *reinterpret_cast<const uint32_t *>(p + 8);
+        const u4 m = {__builtin_amdgcn_alignbit(w[1], w[0], 16), __builtin_amdgcn_alignbit(w[2], w[1], 16),
+                      __builtin_amdgcn_alignbit(w[3], w[2], 16), __builtin_amdgcn_alignbit(w4, w[3], 16)};
+        const u4 e = {w[1], w[2], w[3], w4};
+        acc[3 * dr] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(a, __builtin_bit_cast(b8, w), acc[3 * dr], 0, 0, 0);
+        acc[3 * dr + 1] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(a, __builtin_bit_cast(b8, m), acc[3 * dr + 1], 0, 0, 0);
+        acc[3 * dr + 2] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(a, __builtin_bit_cast(b8, e), acc[3 * dr + 2], 0, 0, 0);
       }
     }
+  }
+  if constexpr (WB == 2) {  // the second half of the rows joins the first
+    f4 *red = reinterpret_cast<f4 *>(sm) + (wv % NB) * 10 * 64 + lane;
     __syncthreads();
+    if (wr == 1) {
+#pragma unroll
+      for (int tap = 0; tap < 9; ++tap) red[tap * 64] = acc[tap];
+      red[9 * 64] = accb;
+    }
+    __syncthreads();
+    if (wr == 1) return;
+#pragma unroll
+    for (int tap = 0; tap < 9; ++tap) acc[tap] += red[tap * 64];
+    accb += red[9 * 64];
   }
   constexpr int NW = 9 * COUT * CIN;
   float *P = part + (size_t)blockIdx.x * (NW + COUT);
 #pragma unroll
   for (int tap = 0; tap < 9; ++tap)
 #pragma unroll
-    for (int co = 0; co < NCO; ++co)
+    for (int e = 0; e < 4; ++e) P[(tap * COUT + co * 16 + 4 * lk + e) * CIN + ci * 16 + lc] = acc[tap][e];
+  if (ci == 0 && lc == 0)
 #pragma unroll
-      for (int ci = 0; ci < NCI; ++ci)
-#pragma unroll
-        for (int e = 0; e < 4; ++e)
-          P[(tap * COUT + co * 16 + 4 * lk + e) * CIN + ci * 16 + lc] = acc[tap][co][ci][e];
-  if (lane < COUT) P[NW + lane] = bacc;
+    for (int e = 0; e < 4; ++e) P[NW + co * 16 + 4 * lk + e] = accb[e];
 }
 
 // Sum of the workgroups' partials (up to 1024 of 9 cout cin + cout floats, 38
 // MB for 32 -> 32 channels).  Bound by the latency of its loads: one thread
 // per sum walking every partial took 202 us (190 GB/s, 37 workgroups); with
 // SP_G groups of partials per sum and SP_U independent running sums per group
-// it takes 5 us (train step, 16 images of 256 x 256: 3338 -> 1368 us).  The order is fixed: partial b goes to group b % SP_G, then
-// the groups' sums are added in order.
+// it takes 5 to 8 us (train step, 16 images of 256 x 256: 3338 -> 1368 us).  The
+// order is fixed: partial b goes to group b % SP_G, then the groups' sums are
+// added in order.
 constexpr int SP_Q = 64, SP_G = 16, SP_U = 4;
 __global__ void __launch_bounds__(SP_Q *SP_G) k_sum_partials(int nblk, int n, const float *__restrict__ part,
                                                              float *__restrict__ dw, int nw, float *__restrict__ db) {
@@ -360,7 +379,8 @@ __global__ void __launch_bounds__(SP_Q *SP_G) k_sum_partials(int nblk, int n, co
 __global__ void __launch_bounds__(256) k_pool(LevelView F, LevelView C, const uint16_t *__restrict__ x,
                                               uint16_t *__restrict__ y) {
   NET_PIXEL8(C)
-  const NImg cm = C.img[t.img], fm = F.img[t.img];
+  const NImg fm = F.img[t.img];
+  const NTile &cm = t;
   if (r >= cm.rows || c >= cm.cols) return;
   const long long q = cm.off + (long long)r * cm.cols + c;
   float s[4] = {0.0f, 0.0f, 0.0f, 0.0f};
@@ -384,7 +404,8 @@ __global__ void __launch_bounds__(256) k_pool(LevelView F, LevelView C, const ui
 __global__ void __launch_bounds__(256) k_upadd(LevelView F, LevelView C, const uint16_t *__restrict__ a,
                                                const uint16_t *__restrict__ b, uint16_t *__restrict__ y) {
   NET_PIXEL8(F)
-  const NImg fm = F.img[t.img], cm = C.img[t.img];
+  const NImg cm = C.img[t.img];
+  const NTile &fm = t;
   if (r >= fm.rows || c >= fm.cols) return;
   const long long p = fm.off + (long long)r * fm.cols + c;
   const long long q = cm.off + (long long)(r >> 1) * cm.cols + (c >> 1);
@@ -399,7 +420,7 @@ __global__ void __launch_bounds__(256) k_gpool(LevelView F, LevelView C, const u
                                                const uint16_t *__restrict__ pc, const uint16_t *__restrict__ yact,
                                                uint16_t *__restrict__ g) {
   NET_PIXEL8(F)
-  const NImg fm = F.img[t.img];
+  const NTile &fm = t;
   if (r >= fm.rows || c >= fm.cols) return;
   const long long p = fm.off + (long long)r * fm.cols + c;
   const s4 ya = ld4(yact + p * 32 + k);
@@ -421,7 +442,8 @@ __global__ void __launch_bounds__(256) k_gpool(LevelView F, LevelView C, const u
 __global__ void __launch_bounds__(256) k_gup(LevelView F, LevelView C, const uint16_t *__restrict__ a,
                                              const uint16_t *__restrict__ yact, uint16_t *__restrict__ g) {
   NET_PIXEL8(C)
-  const NImg cm = C.img[t.img], fm = F.img[t.img];
+  const NImg fm = F.img[t.img];
+  const NTile &cm = t;
   if (r >= cm.rows || c >= cm.cols) return;
   const long long q = cm.off + (long long)r * cm.cols + c;
   float s[4] = {0.0f, 0.0f, 0.0f, 0.0f};
@@ -455,7 +477,7 @@ __global__ void __launch_bounds__(256) k_loss(LevelView L, const float *__restri
   const int wid = blockIdx.x * 4 + (threadIdx.x >> 6);
   if (wid < L.ntiles) {
     const NTile t = L.tiles[wid];
-    const NImg im = L.img[t.img];
+    const NTile &im = t;
     const int r = t.r0 + (lane >> 4), c = t.c0 + (lane & 15);
     if (r < im.rows && c < im.cols) {
       const long long p = im.off + (long long)r * im.cols + c;
@@ -512,18 +534,20 @@ namespace net {
 bool conv(hipStream_t s, const LevelView &L, int cin, int cout, const uint16_t *x, const uint16_t *w,
           const float *bias, int relu, void *y, int yf32) {
   if (L.ntiles == 0) return true;
-  // persistent waves: at most 2048 workgroups, each wavefront strides over the tiles
-  const int nb = std::min(nblk4(L.ntiles), 2048);
-  if (cin == 16 && cout == 32 && !yf32)
-    hipLaunchKernelGGL((k_conv<16, 32, false>), dim3(nb), dim3(256), 0, s, L.img, L.tiles, L.ntiles, x, w, bias, relu, y);
-  else if (cin == 32 && cout == 32 && !yf32)
-    hipLaunchKernelGGL((k_conv32<32, false>), dim3(nb), dim3(256), 0, s, L.img, L.tiles, L.ntiles, x, w, bias, relu, y);
-  else if (cin == 32 && cout == 16 && yf32)
-    hipLaunchKernelGGL((k_conv32<16, true>), dim3(nb), dim3(256), 0, s, L.img, L.tiles, L.ntiles, x, w, bias, relu, y);
-  else if (cin == 32 && cout == 16 && !yf32)
-    hipLaunchKernelGGL((k_conv32<16, false>), dim3(nb), dim3(256), 0, s, L.img, L.tiles, L.ntiles, x, w, bias, relu, y);
-  else
-    return false;
+  // a multiple of 8 workgroups (one run of tiles per XCD), at most as many as
+  // are resident at once (registers: two per CU for 32 -> 32 channels, else
+  // three); more of them load the weights again: 32 -> 32 over 1.3 million
+  // pixels took 40 us with 512, 46 with 768 and 1536, 16 -> 32 took 33 us with
+  // 768, 39 with 512 and 1024
+  const int nb = std::min((nblk4(L.ntiles) + 7) / 8 * 8, cin == 32 && cout == 32 ? 512 : 768);
+#define CONV(CI, CO, F32)                                                                                        \
+  hipLaunchKernelGGL((k_conv<CI, CO, F32>), dim3(nb), dim3(256), 0, s, L.tiles, L.ntiles, x, w, bias, relu, y)
+  if (cin == 16 && cout == 32 && !yf32) CONV(16, 32, false);
+  else if (cin == 32 && cout == 32 && !yf32) CONV(32, 32, false);
+  else if (cin == 32 && cout == 16 && yf32) CONV(32, 16, true);
+  else if (cin == 32 && cout == 16 && !yf32) CONV(32, 16, false);
+  else return false;
+#undef CONV
   return true;
 }
 
@@ -535,11 +559,11 @@ bool conv_dw(hipStream_t s, const LevelView &L, int cin, int cout, const uint16_
   const int n = 9 * cout * cin + cout;
   if (L.ntiles == 0) return false;
   if (cin == 16 && cout == 32)
-    hipLaunchKernelGGL((k_conv_dw<16, 32>), dim3(nb), dim3(64), 0, s, L.img, L.tiles, L.ntiles, g, x, part);
+    hipLaunchKernelGGL((k_conv_dw<16, 32>), dim3(nb), dim3(256), 0, s, L.tiles, L.ntiles, g, x, part);
   else if (cin == 32 && cout == 32)
-    hipLaunchKernelGGL((k_conv_dw<32, 32>), dim3(nb), dim3(64), 0, s, L.img, L.tiles, L.ntiles, g, x, part);
+    hipLaunchKernelGGL((k_conv_dw<32, 32>), dim3(nb), dim3(256), 0, s, L.tiles, L.ntiles, g, x, part);
   else if (cin == 32 && cout == 16)
-    hipLaunchKernelGGL((k_conv_dw<32, 16>), dim3(nb), dim3(64), 0, s, L.img, L.tiles, L.ntiles, g, x, part);
+    hipLaunchKernelGGL((k_conv_dw<32, 16>), dim3(nb), dim3(256), 0, s, L.tiles, L.ntiles, g, x, part);
   else
     return false;
   sum_partials(s, nb, n, part, dw, 9 * cout * cin, db);

@@ -287,3 +287,41 @@ def test_grad_w_partial_counts(env, ntiles):
     assert np.array_equal(dw.cpu().numpy().reshape(9, 32, 32), rw)
     assert np.array_equal(db.cpu().numpy(), rb)
     plan.close()
+
+
+@pytest.mark.parametrize("cin,cout", [(16, 32), (32, 32), (32, 16)])
+@pytest.mark.parametrize("ntiles", [1, 31, 33, 2049, 6150])
+def test_convolutions_over_many_tiles(env, ntiles, cin, cout):
+    """Runs of tiles per XCD, wavefronts that take one tile, several or none, and
+    the look-ahead at a run's end: one ragged image of `ntiles` tiles (and a
+    second one of a pixel).  Integer entries: the sums are exact in FP32 in any
+    order, and the outputs are their one BF16 rounding."""
+    torch, learned, ctx = env
+    rng = np.random.default_rng(ntiles + cin)
+    shp = [(3, 16 * ntiles - 5), (1, 1)]
+    plan = learned.Plan(ctx, rows=[r for r, _ in shp], cols=[c for _, c in shp])
+    xs = [rng.integers(-1, 2, size=(r, c, cin)).astype(np.float64) for r, c in shp]
+    gs = [rng.integers(-1, 2, size=(r, c, cout)).astype(np.float64) for r, c in shp]
+    w = rng.integers(-1, 2, size=(9, cout, cin)).astype(np.float64)
+    b = rng.integers(-2, 3, size=cout).astype(np.float64)
+    L = learned._bind(ctx.L)
+    x_d, g_d, w_d = (dev(torch, bits(a).ravel()) for a in (pack_images(xs), pack_images(gs), w))
+    b_d = dev(torch, b.astype(np.float32))
+    y = torch.zeros(sum(r * c for r, c in shp) * cout, dtype=torch.int16, device="cuda")
+    work = torch.zeros(int(L.imau_net_grad_w_work(plan.h, 0, cin, cout)), dtype=torch.float32, device="cuda")
+    dw = torch.zeros(9 * cout * cin, dtype=torch.float32, device="cuda")
+    db = torch.zeros(cout, dtype=torch.float32, device="cuda")
+    ctx._check(L.imau_net_conv(ctx.h, plan.h, 0, cin, cout, learned._ptr(x_d), learned._ptr(w_d), learned._ptr(b_d),
+                               1, learned._ptr(y), 0))
+    ctx._check(L.imau_net_conv_grad_w(ctx.h, plan.h, 0, cin, cout, learned._ptr(g_d), learned._ptr(x_d),
+                                      learned._ptr(dw), learned._ptr(db), learned._ptr(work)))
+    ctx._check(L.imau_net_sync(ctx.h))
+    rw, rb = np.zeros((9, cout, cin)), np.zeros(cout)
+    for got, x, g in zip(split_images(unbits(y), shp, cout), xs, gs):
+        assert np.array_equal(got, NO.bf16(np.maximum(NO.conv(x, w, b), 0.0)))
+        a, c = NO.conv_grad_w(g, x)
+        rw += a
+        rb += c
+    assert np.array_equal(dw.cpu().numpy().reshape(rw.shape), rw)
+    assert np.array_equal(db.cpu().numpy(), rb)
+    plan.close()
