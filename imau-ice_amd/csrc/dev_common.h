@@ -39,6 +39,16 @@
 #define IMAU_MTI 0
 #define IMAU_MTI_CANDIDATES {0, 4, 8, 16, 32}
 #define IMAU_MNZ 15
+// small-grid viscosity kernel (one wavefront per level): most levels (the
+// wavefronts of a workgroup) and most IMAU_VTI-row tiles.  FP64 DIVA, 15
+// levels, us against the tiled kernel: 8.4 / 16.8 at 6 tiles, 14.9 / 16.7 at
+// 51; then it grows by 0.16 us a tile (109 / 46 at 637), the tiled one stays
+#define IMAU_LEVMAX 16
+#define IMAU_LEVTILES 56
+// workgroups per tile of the tiled kernel: one row per wavefront (us with one
+// and two: 28.6 / 16.7 at 51 tiles, 54 / 46 at 637, both FP64; FP32 40 / 38.5
+// at 1024, 102 / 94 at 3000)
+#define IMAU_VISC_GY (IMAU_VTI / IMAU_WG_I)
 
 // Workgroups are dispatched round-robin over the 8 XCDs (workgroup b on XCD
 // b % 8), each with its own L2.  Tile kernels run tile imau_xcd_tile() rather

@@ -17,6 +17,8 @@
 #define FOR_TILE_ROWS for (int ii = threadIdx.y; ii < IMAU_TI; ii += IMAU_WG_I)
 // one cell at a time, where unrolling would cost more registers than it hides latency
 #define FOR_TILE_ROWS_1 _Pragma("unroll 1") for (int ii = threadIdx.y; ii < IMAU_TI; ii += IMAU_WG_I)
+// with the rows of a tile dealt to gridDim.y workgroups
+#define FOR_VTILE_ROWS_Y _Pragma("unroll 1") for (int ii = threadIdx.y + IMAU_WG_I * blockIdx.y; ii < IMAU_VTI; ii += IMAU_WG_I * gridDim.y)
 #define FOR_VTILE_ROWS _Pragma("unroll 1") for (int ii = threadIdx.y; ii < IMAU_VTI; ii += IMAU_WG_I)
 
 // ---------------------------------------------------------------------------
@@ -471,14 +473,24 @@ __device__ __forceinline__ T visc_level(const ViscCol<T> &c, T z, T vc, T vw, T 
 // trapezoid steps of the viscosity integral and the F2 integrand (H/eta) z^2
 // (vertical_integrate, src/utilities_module.f90:73-96; :960-1013)
 template <class T>
+__device__ __forceinline__ T visc_g(T z, T eta, T HiT) {
+#pragma clang fp contract(off)
+  return wdiv(HiT, eta) * (z * z);
+}
+template <class T>
+__device__ __forceinline__ T visc_add(T sum, T a, T aprev, T z, T zprev) {
+#pragma clang fp contract(off)
+  const T dz = z - zprev;
+  return sum + (T)0.5 * (a + aprev) * dz;
+}
+template <class T>
 __device__ __forceinline__ void visc_trap(int k, T z, T zprev, T eta, T HiT, T &vint, T &F2int, T &eta_prev,
                                           T &g_prev) {
 #pragma clang fp contract(off)
-  const T gk = wdiv(HiT, eta) * (z * z);
+  const T gk = visc_g<T>(z, eta, HiT);
   if (k > 0) {
-    const T dz = z - zprev;
-    vint += (T)0.5 * (eta + eta_prev) * dz;
-    F2int += (T)0.5 * (gk + g_prev) * dz;
+    vint = visc_add<T>(vint, eta, eta_prev, z, zprev);
+    F2int = visc_add<T>(F2int, gk, g_prev, z, zprev);
   }
   eta_prev = eta;
   g_prev = gk;
@@ -493,14 +505,14 @@ __global__ void __launch_bounds__(IMAU_WG) k_visc(const Member *__restrict__ mem
   if (j >= m.ny) return;
   const int nx = m.nx, ny = m.ny, nz = kp.nz;
   if (!active[t.g]) {  // finished member: keep its viscosity in the buffer that becomes current
-    FOR_VTILE_ROWS {
+    FOR_VTILE_ROWS_Y {
       const int i = t.i0 + ii;
       if (i >= nx) break;
       for (int k = 0; k < nz; ++k) visc_out[p3(m, k, j, i)] = visc_in[p3(m, k, j, i)];
     }
     return;
   }
-  FOR_VTILE_ROWS {
+  FOR_VTILE_ROWS_Y {
     const int i = t.i0 + ii;
     if (i >= nx) break;
     const long long p = p2(m, j, i);
@@ -567,6 +579,72 @@ __global__ void __launch_bounds__(IMAU_WG) k_visc(const Member *__restrict__ mem
     }
     // F2 integral (calc_F_integral, :960-1013)
     if (DIVA) f.F2[p] = (mi == 1) ? fmax(kp.F_int_min, (double)F2int) : ((kp.margin == 0) ? 0.0 : kp.F_int_min);
+  }
+}
+
+// The same for small grids, where k_visc leaves the chip idle and its time is
+// one column's chain of levels (a division, a cube root and a round trip to
+// memory each): a workgroup per row of a tile, a wavefront per level; the
+// integrals are summed afterwards from LDS, in the same order with the same
+// rounding, so the results are the same bit for bit.  The column's 25 values
+// are loaded once per level, which costs nothing while the chip is idle.
+// 30 -> 8.4 us on 29x29 cells, 30 -> 15 on 401x41 (FP64, 15 levels).
+template <bool DIVA, bool THIRD, class T>
+__global__ void __launch_bounds__(IMAU_TJ *IMAU_LEVMAX) k_visc_lev(
+    const Member *__restrict__ mem, const Tile *__restrict__ tiles, const KP kp, const Fields f,
+    const T *__restrict__ visc_in, T *__restrict__ visc_out, const T *__restrict__ B3, const int *__restrict__ active) {
+  __shared__ T s_eta[IMAU_LEVMAX][IMAU_TJ], s_g[DIVA ? IMAU_LEVMAX : 1][IMAU_TJ];
+  TILE_SETUP
+  const int nx = m.nx, ny = m.ny, nz = kp.nz;
+  const int i = t.i0 + (int)blockIdx.y, k = __builtin_amdgcn_readfirstlane(threadIdx.y);
+  if (i >= nx) return;  // the whole workgroup
+  const bool in = j < ny;
+  const long long q = p3(m, k, min(j, ny - 1), i);
+  if (!active[t.g]) {
+    if (in) visc_out[q] = visc_in[q];
+    return;
+  }
+  const long long p = p2(m, min(j, ny - 1), i);
+  const double Hi = f.Hi[p];
+  const int mi = f.m_ice[p];
+  const bool bc_skip = (kp.margin == 0 && mi == 0);
+  T eta = (T)0.0;
+  if (in) {
+    T vc = (T)0.0, vw = (T)0.0, ve = (T)0.0, vs = (T)0.0, vn = (T)0.0;
+    if (DIVA) {
+      vc = visc_in[q];
+      vw = visc_in[(i > 0) ? q - ny : q];
+      ve = visc_in[(i < nx - 1) ? q + ny : q];
+      vs = visc_in[(j > 0) ? q - 1 : q];
+      vn = visc_in[(j < ny - 1) ? q + 1 : q];
+    }
+    const T B = B3[q], z = (T)kp.zeta[k];
+    const ViscCol<T> cc = visc_col<DIVA, T>(m, kp, f, j, i, Hi, f.eps_h[p]);
+    if (i == 0) vw = (T)0.0;
+    if (i == nx - 1) ve = (T)0.0;
+    if (j == 0) vs = (T)0.0;
+    if (j == ny - 1) vn = (T)0.0;
+    if (!bc_skip) eta = visc_level<DIVA, THIRD, T>(cc, z, vc, vw, ve, vs, vn, B);
+    visc_out[q] = eta;
+    s_eta[k][threadIdx.x] = eta;
+    if (DIVA) s_g[k][threadIdx.x] = visc_g<T>(z, eta, cc.HiT);
+  }
+  __syncthreads();
+  if (!in) return;
+  const int lx = threadIdx.x;
+  if (k == 0 && !bc_skip) {
+    T vint = (T)0.0;
+    for (int l = 1; l < nz; ++l)
+      vint = visc_add<T>(vint, s_eta[l][lx], s_eta[l - 1][lx], (T)kp.zeta[l], (T)kp.zeta[l - 1]);
+    f.visc_int[p] = (double)vint;
+    f.N_a[p] = (double)vint * ((kp.margin == 0) ? Hi : fmax(0.1, Hi));
+  }
+  if (DIVA && k == (nz > 1 ? 1 : 0)) {
+    T F2int = (T)0.0;
+    if (!bc_skip)
+      for (int l = 1; l < nz; ++l)
+        F2int = visc_add<T>(F2int, s_g[l][lx], s_g[l - 1][lx], (T)kp.zeta[l], (T)kp.zeta[l - 1]);
+    f.F2[p] = (mi == 1) ? fmax(kp.F_int_min, (double)F2int) : ((kp.margin == 0) ? 0.0 : kp.F_int_min);
   }
 }
 
@@ -1797,6 +1875,22 @@ void setup1(const Launch &L, const KP &kp, const Fields &f, const double *yg) {
 void setup2(const Launch &L, const KP &kp, const Fields &f) {
   hipLaunchKernelGGL(k_setup2, dim3(L.ntiles), wg(), 0, L.s, L.mem, L.tiles, kp, f);
 }
+template <class T>
+static void visc_tiles(const Launch &L, const Launch &LV, const KP &kp, const Fields &f, bool diva, const T *visc_in,
+                       T *visc_out, const T *B3, const int *active) {
+  const bool third = kp.n_flow == 3.0;
+  // few tiles: a wavefront per level instead of per column (the line's two sides stand at IMAU_LEVTILES)
+  if (kp.nz <= IMAU_LEVMAX && LV.ntiles <= IMAU_LEVTILES) {
+    auto kl = diva ? (third ? k_visc_lev<true, true, T> : k_visc_lev<true, false, T>)
+                   : (third ? k_visc_lev<false, true, T> : k_visc_lev<false, false, T>);
+    hipLaunchKernelGGL(kl, dim3(LV.ntiles, IMAU_VTI), dim3(IMAU_TJ, kp.nz), 0, L.s, L.mem, LV.tiles, kp, f, visc_in,
+                       visc_out, B3, active);
+    return;
+  }
+  auto kv = diva ? (third ? k_visc<true, true, T> : k_visc<true, false, T>)
+                 : (third ? k_visc<false, true, T> : k_visc<false, false, T>);
+  hipLaunchKernelGGL(kv, dim3(LV.ntiles, IMAU_VISC_GY), wg(), 0, L.s, L.mem, LV.tiles, kp, f, visc_in, visc_out, B3, active);
+}
 void visc3d(const Launch &L, const Launch &LV, const KP &kp, const Fields &f, bool diva, const double *visc_in,
             double *visc_out, const int *active) {
   // n = 3 (every shipped configuration) takes the cube-root form of the viscosity
@@ -1808,10 +1902,8 @@ void visc3d(const Launch &L, const Launch &LV, const KP &kp, const Fields &f, bo
                        active);
     return;
   }
-  auto kv = diva ? (third ? k_visc<true, true, double> : k_visc<true, false, double>)
-                 : (third ? k_visc<false, true, double> : k_visc<false, false, double>);
   hipLaunchKernelGGL(k_strain, dim3(L.ntiles), wg(), 0, L.s, L.mem, L.tiles, kp, f, active);
-  hipLaunchKernelGGL(kv, dim3(LV.ntiles), wg(), 0, L.s, L.mem, LV.tiles, kp, f, visc_in, visc_out, f.B3, active);
+  visc_tiles<double>(L, LV, kp, f, diva, visc_in, visc_out, f.B3, active);
 }
 void visc3d32(const Launch &L, const Launch &LV, const KP &kp, const Fields &f, bool diva, const float *visc_in,
               float *visc_out, const float *B3, const int *active) {
@@ -1822,10 +1914,8 @@ void visc3d32(const Launch &L, const Launch &LV, const KP &kp, const Fields &f, 
     hipLaunchKernelGGL(km, dim3(LV.nmtiles), dim3(64), 0, L.s, L.mem, LV.mtiles, kp, f, visc_in, visc_out, B3, active);
     return;
   }
-  auto kv = diva ? (third ? k_visc<true, true, float> : k_visc<true, false, float>)
-                 : (third ? k_visc<false, true, float> : k_visc<false, false, float>);
   hipLaunchKernelGGL(k_strain, dim3(L.ntiles), wg(), 0, L.s, L.mem, L.tiles, kp, f, active);
-  hipLaunchKernelGGL(kv, dim3(LV.ntiles), wg(), 0, L.s, L.mem, LV.tiles, kp, f, visc_in, visc_out, B3, active);
+  visc_tiles<float>(L, LV, kp, f, diva, visc_in, visc_out, B3, active);
 }
 __global__ void k_d2f(const double *__restrict__ a, float *__restrict__ b, long long n) {
   for (long long q = blockIdx.x * (long long)blockDim.x + threadIdx.x; q < n; q += (long long)gridDim.x * blockDim.x)

@@ -55,6 +55,32 @@ def test_every_tile_height_gives_the_same_solve(ctx, precision):
                 np.testing.assert_array_equal(st[m][f], st0[m][f], err_msg="%s %s member %d" % (key, f, m))
 
 
+@pytest.mark.parametrize("precision", ["fp64", "mixed_visc"])
+@pytest.mark.parametrize("shape,nz,dyn,n_flow", [((9, 12), 15, "DIVA", 3.0), ((9, 64), 16, "DIVA", 3.0),
+                                                 ((17, 65), 2, "DIVA", 2.5), ((8, 129), 15, "SSA", 3.0),
+                                                 ((26, 40), 5, "SSA", 2.5)])
+def test_viscosity_by_level_equals_by_column(ctx, shape, nz, dyn, n_flow, precision):
+    """A few tiles take one wavefront per level, many one lane per column: a
+    small member solved alone and beside a large one (1, 2 and 3 tile columns,
+    the fewest and most levels) ends in the same state bit for bit."""
+    z = np.linspace(0.0, 1.0, nz) ** 0.8
+    cfg = geometry.synthetic_config(choice_ice_dynamics=dyn, n_flow=n_flow, zeta=[float(a) for a in z])
+    config.set_config(cfg, stop_rule=1, nonlinear_rtol=1e-12, DIVA_visc_it_nit=4, precision=precision)
+    g1, _, s1 = geometry.random_geometry(*shape, seed=3, cfg=cfg)
+    g2, _, s2 = geometry.random_geometry(330, 130, seed=4, cfg=cfg)
+    out = []
+    for grids, states in (([g1], [s1.copy()]), ([g1, g2], [s1.copy(), s2.copy()])):
+        prob = solver.Problem(ctx, grids, cfg, states)
+        try:
+            prob.solve(cfg)
+            out.append(prob.download()[0].copy())
+        finally:
+            prob.close()
+    assert np.abs(out[0]["u_vav_cx"]).max() > 0.0
+    for f in ("u_vav_cx", "v_vav_cy", "visc_eff_3D_a", "N_a") + (("F2_a",) if dyn == "DIVA" else ()):
+        np.testing.assert_array_equal(out[0][f], out[1][f], err_msg=f)
+
+
 def test_tile_height_outside_the_candidates_is_rejected(ctx):
     g, cfg, st = geometry.dome()
     prob = solver.Problem(ctx, [g], cfg, [st])
