@@ -15,8 +15,6 @@
   const int j = t.j0 + (int)threadIdx.x;
 
 #define FOR_TILE_ROWS for (int ii = threadIdx.y; ii < IMAU_TI; ii += IMAU_WG_I)
-// one cell at a time, where unrolling would cost more registers than it hides latency
-#define FOR_TILE_ROWS_1 _Pragma("unroll 1") for (int ii = threadIdx.y; ii < IMAU_TI; ii += IMAU_WG_I)
 // with the rows of a tile dealt to gridDim.y workgroups
 #define FOR_VTILE_ROWS_Y _Pragma("unroll 1") for (int ii = threadIdx.y + IMAU_WG_I * blockIdx.y; ii < IMAU_VTI; ii += IMAU_WG_I * gridDim.y)
 #define FOR_VTILE_ROWS _Pragma("unroll 1") for (int ii = threadIdx.y; ii < IMAU_VTI; ii += IMAU_WG_I)
@@ -1001,85 +999,6 @@ __device__ __forceinline__ void v_row(const Member &m, const KP &kp, const CoefP
 
 
 
-// The rows of one cell at the vectors (xu, xv): S and D of its u and v unknown,
-// from the loaded neighbourhood; only 'infinite' and 'periodic' boundary rows
-// read one more value, their source.
-__device__ __forceinline__ bool zero_row(uint8_t rt) { return rt == RT_ZERO || rt == RT_BND_ZERO; }
-__device__ __forceinline__ bool copy_row(uint8_t rt) { return rt == RT_BND_INF || rt == RT_BND_PER; }
-template <int CROSS>
-struct CellRows {
-  Hood<double> U, V;
-  HoodCoef<double> k;
-  uint8_t ru, rv;
-  __device__ __forceinline__ bool hu(const Member &m) const { return k.i < m.nx - 1; }  // the cell has a u unknown
-  __device__ __forceinline__ bool hv(const Member &m) const { return k.j < m.ny - 1; }
-  __device__ __forceinline__ void load(const Member &m, const CoefP &c, const double *xu, const double *xv, int j,
-                                       int i) {
-    const uint32_t p = (uint32_t)i * (uint32_t)m.ny + (uint32_t)j;
-    ru = (c.rt_u + m.off)[p];
-    rv = (c.rt_v + m.off)[p];
-    hood_load<double, CROSS>(m, c, xu, xv, j, i, U, V, k);
-  }
-  // the source of a boundary row that copies one
-  __device__ __forceinline__ long long u_src(const Member &m) const {
-    int jo, io;
-    bnd_src(ru, k.i, k.j, m.nx - 2, m.ny - 1, jo, io);
-    return p2(m, jo, io);
-  }
-  __device__ __forceinline__ long long v_src(const Member &m) const {
-    int jo, io;
-    bnd_src(rv, k.i, k.j, m.nx - 1, m.ny - 2, jo, io);
-    return p2(m, jo, io);
-  }
-  // interior and calving-front rows
-  __device__ __forceinline__ void u_in(const Member &m, const KP &kp, double &S, double &D) const {
-    u_sd_x<CROSS, double>(m, kp, k, k.j, k.i, ru, U, V, S, D);
-  }
-  __device__ __forceinline__ void v_in(const Member &m, const KP &kp, double &S, double &D) const {
-    v_sd_x<CROSS, double>(m, kp, k, k.j, k.i, rv, U, V, S, D);
-  }
-  __device__ __forceinline__ void u_sd(const Member &m, const KP &kp, const double *xu, double &S, double &D) const {
-    if (in_row(ru)) { u_in(m, kp, S, D); return; }
-    S = copy_row(ru) ? -xu[u_src(m)] : 0.0;
-    D = 1.0;
-  }
-  __device__ __forceinline__ void v_sd(const Member &m, const KP &kp, const double *xv, double &S, double &D) const {
-    if (in_row(rv)) { v_in(m, kp, S, D); return; }
-    S = copy_row(rv) ? -xv[v_src(m)] : 0.0;
-    D = 1.0;
-  }
-};
-// right-hand sides of the rows (tau: the driving stress at the row; ns: N on its
-// own grid, in the form without cross terms)
-template <int CROSS>
-__device__ __forceinline__ double u_rhs(const Member &m, const CoefP &c, int j, int i, uint8_t rt, double tau,
-                                        double ns) {
-  if (rt == RT_FREE) {
-    const double b = -tau * (m.dx * m.dx);
-    return CROSS ? b : b / ns;
-  }
-  if (rt == RT_MARGIN_I || rt == RT_MARGIN_O) return c.frhs[p2(m, j, (rt == RT_MARGIN_I) ? i : i + 1)];
-  return 0.0;
-}
-template <int CROSS>
-__device__ __forceinline__ double v_rhs(const Member &m, const CoefP &c, int j, int i, uint8_t rt, double tau,
-                                        double ns) {
-  if (rt == RT_FREE) {
-    const double b = -tau * (m.dx * m.dx);
-    return CROSS ? b : b / ns;
-  }
-  if (rt == RT_MARGIN_I || rt == RT_MARGIN_O) return c.frhs[p2(m, (rt == RT_MARGIN_I) ? j : j + 1, i)];
-  return 0.0;
-}
-// The operator kernels (k_apply, k_resid, k_bicg_init) are bound
-// by load latency at small sizes and by how many loads are in flight at large
-// ones: the some 25 values of a cell are all loaded before its rows are
-// evaluated.  (Both of a thread's cells at once took more registers than the
-// extra loads in flight were worth.)  k_apply 7.0 -> 5.1 us on the 401x41
-// channel (FP64), 23.4 -> 18.8 on 12 ice caps of 96 to 512 a side
-// (FP32 operator), k_bicg_init 9.6 -> 6.2, k_resid 6.7 -> 5.6.  k_resid_init
-// keeps its look-ups: loaded first it took 54 instead of 70 us on the 12 caps,
-// but 30 instead of 27 on 8 of 256x256.
 constexpr int TROWS = IMAU_TI / IMAU_WG_I;
 
 // ---------------------------------------------------------------------------
@@ -1380,32 +1299,28 @@ __global__ void __launch_bounds__(IMAU_WG) k_net_warm(const Member *__restrict__
 
 // FP64 residual partial sums: sum (S + D x - b)^2 and sum b^2 over every row
 // of the system assembled at the current coefficients.
-template <int CROSS>
 __global__ void __launch_bounds__(IMAU_WG) k_resid(const Member *__restrict__ mem, const Tile *__restrict__ tiles,
                                                    const KP kp, const CoefP c, const double *__restrict__ xu,
                                                    const double *__restrict__ xv, double *__restrict__ partial) {
   TILE_SETUP
   double acc[2] = {0.0, 0.0};
-  if (j < m.ny) {
-    FOR_TILE_ROWS_1 {
+  const int nx = m.nx, ny = m.ny;
+  const GAcc U{xu, m}, V{xv, m};
+  if (j < ny) {
+    FOR_TILE_ROWS {
       const int i = t.i0 + ii;
-      if (i >= m.nx) break;
-      CellRows<CROSS> cr;
-      cr.load(m, c, xu, xv, j, i);
-      const double tu = c.taudx[p2(m, j, i)];
-      const double tv = c.taudy[p2(m, j, i)];
-      double S, D;
-      if (cr.hu(m)) {
-        cr.u_sd(m, kp, xu, S, D);
-        const double b = u_rhs<CROSS>(m, c, j, i, cr.ru, tu, cr.k.nb0);
-        const double r = S + D * cr.U.c - b;
+      if (i >= nx) break;
+      const long long p = p2(m, j, i);
+      double S, D, b;
+      if (i < nx - 1) {
+        u_row(m, kp, c, j, i, c.rt_u[p], U, V, S, D, b);
+        const double r = S + D * xu[p] - b;
         acc[0] += r * r;
         acc[1] += b * b;
       }
-      if (cr.hv(m)) {
-        cr.v_sd(m, kp, xv, S, D);
-        const double b = v_rhs<CROSS>(m, c, j, i, cr.rv, tv, cr.k.nbw);
-        const double r = S + D * cr.V.c - b;
+      if (j < ny - 1) {
+        v_row(m, kp, c, j, i, c.rt_v[p], U, V, S, D, b);
+        const double r = S + D * xv[p] - b;
         acc[0] += r * r;
         acc[1] += b * b;
       }
@@ -1987,8 +1902,7 @@ void post(const Launch &L, const KP &kp, const Fields &f, const double *xu, cons
                      relax, mix);
 }
 void resid(const Launch &L, const KP &kp, const Coef &c, const double *xu, const double *xv, double *partial) {
-  auto k = kp.cross ? k_resid<1> : k_resid<0>;
-  hipLaunchKernelGGL(k, dim3(L.ntiles), wg(), 0, L.s, L.mem, L.tiles, kp, to_p(c), xu, xv, partial);
+  hipLaunchKernelGGL(k_resid, dim3(L.ntiles), wg(), 0, L.s, L.mem, L.tiles, kp, to_p(c), xu, xv, partial);
 }
 void member_sum3(hipStream_t s, int ngrids, const int *tstart, const double *partial, double *out) {
   hipLaunchKernelGGL(k_member_sum<3>, dim3(ngrids), dim3(256), 0, s, tstart, partial, out);
@@ -2080,29 +1994,24 @@ __global__ void __launch_bounds__(IMAU_WG) k_apply(const Member *__restrict__ me
                                                    const int *__restrict__ active, double *__restrict__ partial) {
   TILE_SETUP
   double acc[2] = {0.0, 0.0};
+  const GAcc U{x.u, m}, V{x.v, m};
   if (j < m.ny && active[t.g]) {
-    FOR_TILE_ROWS_1 {
+    FOR_TILE_ROWS {
       const int i = t.i0 + ii;
       if (i >= m.nx) break;
-      CellRows<CROSS> cr;
-      cr.load(m, c, x.u, x.v, j, i);
-      const double wu = w.u ? w.u[p2(m, j, i)] : 0.0;
-      const double wv = w.u ? w.v[p2(m, j, i)] : 0.0;
       const long long p = p2(m, j, i);
       double S, D;
-      if (cr.hu(m)) {
-        cr.u_sd(m, kp, x.u, S, D);
-        const double yv = S + D * cr.U.c;
+      if (i < m.nx - 1) {
+        u_sd_x<CROSS, double>(m, kp, c, j, i, c.rt_u[p], U, V, S, D);
+        const double yv = S + D * x.u[p];
         y.u[p] = yv;
-        acc[0] += wu * yv;
-        acc[1] += yv * yv;
+        if (w.u) { acc[0] += w.u[p] * yv; acc[1] += yv * yv; }
       }
-      if (cr.hv(m)) {
-        cr.v_sd(m, kp, x.v, S, D);
-        const double yv = S + D * cr.V.c;
+      if (j < m.ny - 1) {
+        v_sd_x<CROSS, double>(m, kp, c, j, i, c.rt_v[p], U, V, S, D);
+        const double yv = S + D * x.v[p];
         y.v[p] = yv;
-        acc[0] += wv * yv;
-        acc[1] += yv * yv;
+        if (w.u) { acc[0] += w.v[p] * yv; acc[1] += yv * yv; }
       }
     }
   }
@@ -2110,35 +2019,29 @@ __global__ void __launch_bounds__(IMAU_WG) k_apply(const Member *__restrict__ me
 }
 
 // r = b - A x, rhat = r, p = v = 0; partials (r, r), (b, b)
-template <int CROSS>
 __global__ void __launch_bounds__(IMAU_WG) k_bicg_init(const Member *__restrict__ mem, const Tile *__restrict__ tiles,
                                                        const KP kp, const CoefP c, CVec2 x, Vec2 r, Vec2 rh, Vec2 pp,
                                                        Vec2 vv, const int *__restrict__ active,
                                                        double *__restrict__ partial) {
   TILE_SETUP
   double acc[2] = {0.0, 0.0};
+  const GAcc U{x.u, m}, V{x.v, m};
   if (j < m.ny && active[t.g]) {
-    FOR_TILE_ROWS_1 {
+    FOR_TILE_ROWS {
       const int i = t.i0 + ii;
       if (i >= m.nx) break;
-      CellRows<CROSS> cr;
-      cr.load(m, c, x.u, x.v, j, i);
-      const double tu = c.taudx[p2(m, j, i)];
-      const double tv = c.taudy[p2(m, j, i)];
       const long long p = p2(m, j, i);
-      double S, D;
-      if (cr.hu(m)) {
-        cr.u_sd(m, kp, x.u, S, D);
-        const double b = u_rhs<CROSS>(m, c, j, i, cr.ru, tu, cr.k.nb0);
-        const double rv = b - (S + D * cr.U.c);
+      double S, D, b;
+      if (i < m.nx - 1) {
+        u_row(m, kp, c, j, i, c.rt_u[p], U, V, S, D, b);
+        const double rv = b - (S + D * x.u[p]);
         r.u[p] = rv;
         if (rh.u) { rh.u[p] = rv; pp.u[p] = 0.0; vv.u[p] = 0.0; }
         acc[0] += rv * rv; acc[1] += b * b;
       }
-      if (cr.hv(m)) {
-        cr.v_sd(m, kp, x.v, S, D);
-        const double b = v_rhs<CROSS>(m, c, j, i, cr.rv, tv, cr.k.nbw);
-        const double rv = b - (S + D * cr.V.c);
+      if (j < m.ny - 1) {
+        v_row(m, kp, c, j, i, c.rt_v[p], U, V, S, D, b);
+        const double rv = b - (S + D * x.v[p]);
         r.v[p] = rv;
         if (rh.u) { rh.v[p] = rv; pp.v[p] = 0.0; vv.v[p] = 0.0; }
         acc[0] += rv * rv; acc[1] += b * b;
@@ -2430,8 +2333,7 @@ void apply(const Launch &L, const KP &kp, const Coef &c, const double *xu, const
 void bicg_init(const Launch &L, const KP &kp, const Coef &c, const double *xu, const double *xv, double *ru, double *rv,
                double *rhu, double *rhv, double *pu, double *pv, double *vu, double *vv, const int *active,
                double *partial) {
-  auto k = kp.cross ? k_bicg_init<1> : k_bicg_init<0>;
-  hipLaunchKernelGGL(k, dim3(L.ntiles), wg(), 0, L.s, L.mem, L.tiles, kp, to_p(c), CVec2{xu, xv}, Vec2{ru, rv},
+  hipLaunchKernelGGL(k_bicg_init, dim3(L.ntiles), wg(), 0, L.s, L.mem, L.tiles, kp, to_p(c), CVec2{xu, xv}, Vec2{ru, rv},
                      Vec2{rhu, rhv}, Vec2{pu, pv}, Vec2{vu, vv}, active, partial);
 }
 void bicg_p(const Launch &L, const double *ru, const double *rv, double *pu, double *pv, const double *vu,

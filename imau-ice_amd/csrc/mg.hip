@@ -184,7 +184,7 @@ __device__ __forceinline__ bool fine_valid(const Member &m, int comp, int j, int
 // per cell walked its eight rows and their couplings in turn (34-48 us, whatever
 // the size); here eight lanes share a cell (component x fine row), a row's
 // couplings are gathered first so that their loads are in flight together, and
-// the four rows' sums are added across lanes in the rows' order: 10.7 us on the
+// four lanes add the slots of a component, in the order of the rows: 10.7 us on the
 // 401 x 41 channel (36 before), 14.6 us on 12 caps of 96-512 cells (46 before).
 template <class T, int CROSS>
 __global__ void __launch_bounds__(256) k_gal0_list(const Member *__restrict__ mem, const KP kp, const CoefT<double> c,
@@ -199,15 +199,17 @@ __global__ void __launch_bounds__(256) k_gal0_list(const Member *__restrict__ me
   const int I = e.y / cm.ny, J = e.y - I * cm.ny;
   const long long pc = cm.off + e.y;
   const bool own = (idx >> 3) < n && active[e.x] && cvalid(cm, comp, J, I) && !((plain[pc] >> comp) & 1);
-  double cf[9] = {0, 0, 0, 0, 0, 0, 0, 0, 0};
+  double val[9];
+  int slot[9];
+#pragma unroll
+  for (int k = 0; k < 9; ++k) { val[k] = 0.0; slot[k] = -1; }
   const int j = 2 * J + dj, i = 2 * I + di;
   if (own && fine_valid(m, comp, j, i)) {
     const uint8_t rt = comp == 0 ? c.rt_u[p2(m, j, i)] : c.rt_v[p2(m, j, i)];
     if (in_row(rt)) {
       int cc[9], jj[9], ii[9], num = 0;
-      double val[9];
 #pragma unroll
-      for (int k = 0; k < 9; ++k) { cc[k] = comp; jj[k] = j; ii[k] = i; val[k] = 0.0; }
+      for (int k = 0; k < 9; ++k) { cc[k] = comp; jj[k] = j; ii[k] = i; }
       auto put = [&](int c2, int oj, int oi, double v) {
         cc[num] = c2; jj[num] = j + oj; ii[num] = i + oi; val[num] = v;
         ++num;
@@ -226,22 +228,27 @@ __global__ void __launch_bounds__(256) k_gal0_list(const Member *__restrict__ me
           ii[k] = io;
           rk[k] = (cc[k] == 0 ? c.rt_u : c.rt_v)[p2(m, jo, io)];
         }
-        const int s = in_row(rk[k]) ? agg_slot(comp, cc[k], (jj[k] >> 1) - J, (ii[k] >> 1) - I) : -1;
-#pragma unroll
-        for (int q = 0; q < 9; ++q) cf[q] += (q == s) ? val[k] : 0.0;
+        slot[k] = in_row(rk[k]) ? agg_slot(comp, cc[k], (jj[k] >> 1) - J, (ii[k] >> 1) - I) : -1;
       }
     }
   }
+  // lane a of the four sums the slots a, a + 4, a + 8, over the rows in the
+  // order (dj, di) = (0,0), (0,1), (1,0), (1,1) and each row's couplings in turn
+  const int a = idx & 3;
+  double sum[3] = {0.0, 0.0, 0.0};
+#pragma unroll
+  for (int row = 0; row < 4; ++row)
+#pragma unroll
+    for (int k = 0; k < 9; ++k) {
+      const double v = __shfl(val[k], row, 4);
+      const int s = __shfl(slot[k], row, 4);
+#pragma unroll
+      for (int n = 0; n < 3; ++n) sum[n] += (s == a + 4 * n) ? v : 0.0;
+    }
   T *dst = comp == 0 ? L.cu : L.cv;
 #pragma unroll
-  for (int k = 0; k < 9; ++k) {
-    // the rows' order (dj, di) = (0,0), (0,1), (1,0), (1,1)
-    double s = __shfl(cf[k], 0, 4);
-    s += __shfl(cf[k], 1, 4);
-    s += __shfl(cf[k], 2, 4);
-    s += __shfl(cf[k], 3, 4);
-    if (own && (idx & 3) == 0) dst[k * L.na + pc] = (T)s;
-  }
+  for (int n = 0; n < 3; ++n)
+    if (own && a + 4 * n < 9) dst[(a + 4 * n) * L.na + pc] = (T)sum[n];
 }
 
 // Plain aggregates: all four fine rows of a level-1 aggregate of component
@@ -665,19 +672,20 @@ __global__ void __launch_bounds__(IMAU_WG) k_cprolong(CLevelT<T> Fl, CLevelT<T> 
 //     member needs;
 //   - a colour updated twice in a row (the turning points of the symmetric
 //     sweeps) keeps its values, so it is updated once: 6 nsweeps + 1 phases for 8 nsweeps;
-//   - the rows are divided by their diagonal beforehand and summed in two
-//     halves, and a halo of zeros in LDS replaces the bounds tests.
-// 401 x 41 channel (26 x 3 cells, FP64): 19.8 -> 9.7 us; 12 caps of 96-512
+//   - in FP32 the rows are divided by their diagonal beforehand and summed in
+//     two halves (in FP64 that would change the rounding of the solves, which a
+//     time loop can amplify), and a halo of zeros in LDS replaces the bounds tests.
+// 401 x 41 channel (26 x 3 cells, FP64): 19.8 -> 14.7 us (9.7 with divided
+// rows); 12 caps of 96-512
 // cells (up to 32 x 32, FP32): 18.9 -> 12.2 us.
 constexpr int CL = IMAU_CMAX + 2;  // LDS row length, one-cell halo
 
-__device__ __forceinline__ float recip(float D) { return __builtin_amdgcn_rcpf(D); }
-__device__ __forceinline__ double recip(double D) { return 1.0 / D; }
-
-// a row divided by its diagonal: x = b - sum_k cf[k] x_k (zero where the diagonal is)
+// FP32: a row divided by its diagonal, x = b - sum_k cf[k] x_k (zero where the
+// diagonal is); FP64: the row itself, x = (b - sum_k cf[k] x_k) / D, summed and
+// divided as the other smoothers do
 template <class T>
 struct CoarseRow {
-  T cf[8], b;
+  T cf[8], b, D;  // D: FP64 rows only
   int l;       // LDS index, -1: no row
   long long p;
 };
@@ -689,16 +697,29 @@ __device__ __forceinline__ void coarse_row_load(const CLevelT<T> &L, const CMemb
   if (!in || !cvalid(m, COMP, J, I)) return;
   r.p = cp2(m, J, I);
   const T *src = COMP == 0 ? L.cu : L.cv;
-  const T D = src[r.p], inv = D != (T)0.0 ? recip(D) : (T)0.0;
+  const T D = src[r.p];
+  const T inv = sizeof(T) == 8 ? (T)1.0 : D != (T)0.0 ? (T)__builtin_amdgcn_rcpf((float)D) : (T)0.0;
 #pragma unroll
   for (int k = 0; k < 8; ++k) r.cf[k] = src[(k + 1) * L.na + r.p] * inv;
   r.b = (COMP == 0 ? L.bu : L.bv)[r.p] * inv;
+  r.D = D;
   r.l = (I + 1) * CL + J + 1;
 }
 
 template <class T, int COMP>
 __device__ __forceinline__ void coarse_row_gs(const CoarseRow<T> &r, T *su, T *sv) {
   if (r.l < 0) return;
+  if constexpr (sizeof(T) == 8) {
+    T S = (T)0.0;
+#pragma unroll
+    for (int k = 0; k < 8; ++k) {
+      int cc, dj, di;
+      slot_pos(COMP, k + 1, 0, 0, cc, dj, di);
+      S += r.cf[k] * (cc == 0 ? su : sv)[r.l + di * CL + dj];
+    }
+    (COMP == 0 ? su : sv)[r.l] = (r.D != (T)0.0) ? mdiv(r.b - S, r.D) : (T)0.0;
+    return;
+  }
   T s[2] = {r.b, (T)0.0};
 #pragma unroll
   for (int k = 0; k < 8; ++k) {

@@ -129,66 +129,3 @@ __device__ __forceinline__ void v_sd(const Member &m, const KP &kp, const C &c, 
                                      const AU &U, const AV &V, T &S, T &D) {
   v_sd_x<-1, T>(m, kp, c, j, i, rt, U, V, S, D);
 }
-
-// The neighbourhood of one cell in registers: everything the interior and
-// calving-front rows of its u and v unknown read.  All loads are issued before any is used
-// (indices past the slab's edges are clamped: such values belong to boundary
-// rows), where the rows on their own load behind the test of their
-// type, one after the other.  The accessors are what u_sd_x / v_sd_x call, so
-// the arithmetic is the same.
-template <class T>
-struct Hood {
-  T c, e, w, n, s, d;  // d: the diagonal neighbour (u: (j+1, i-1), v: (j-1, i+1))
-  int j, i;
-  __device__ __forceinline__ T operator()(int jj, int ii) const {
-    if (jj == j) return ii == i ? c : (ii == i + 1 ? e : w);
-    if (ii == i) return jj == j + 1 ? n : s;
-    return d;
-  }
-};
-template <class T>
-struct HoodCoef {
-  T na0, nae, nan_, nb0, nbs, nbw, bu, bv;  // N_a at (j,i), (j,i+1), (j+1,i); N_b at (j,i), (j-1,i), (j,i-1)
-  int j, i;
-  __device__ __forceinline__ T na(const Member &, int jj, int ii) const {
-    return ii == i + 1 ? nae : (jj == j + 1 ? nan_ : na0);
-  }
-  __device__ __forceinline__ T nb(const Member &, int jj, int ii) const {
-    return jj == j - 1 ? nbs : (ii == i - 1 ? nbw : nb0);
-  }
-  __device__ __forceinline__ T bx(const Member &, int, int) const { return bu; }
-  __device__ __forceinline__ T by(const Member &, int, int) const { return bv; }
-  // the form without cross terms: N on cx / cy in nb0 / nbw (no N_b is read then)
-  __device__ __forceinline__ T ncx(const Member &, int, int) const { return nb0; }
-  __device__ __forceinline__ T ncy(const Member &, int, int) const { return nbw; }
-};
-// The slab's base is the same for the whole workgroup (a scalar) and offsets in
-// it are 32-bit (a grid of 2^29 cells would need 1.6 TB), so that a load takes
-// one register for its address.
-template <class T, int CROSS>
-__device__ __forceinline__ void hood_load(const Member &m, const CoefT<T> &c, const T *__restrict__ xu,
-                                          const T *__restrict__ xv, int j, int i, Hood<T> &U, Hood<T> &V,
-                                          HoodCoef<T> &k) {
-  const uint32_t ny = (uint32_t)m.ny, p = (uint32_t)i * ny + (uint32_t)j;
-  const uint32_t up = j < m.ny - 1 ? p + 1 : p, dn = j > 0 ? p - 1 : p;
-  const uint32_t rt = i < m.nx - 1 ? p + ny : p, lf = i > 0 ? p - ny : p;
-  const T *u = xu + m.off, *v = xv + m.off, *na = c.Na + m.off;
-  U = Hood<T>{u[p], u[rt], u[lf], u[up], u[dn], u[up + lf - p], j, i};
-  V = Hood<T>{v[p], v[rt], v[lf], v[up], v[dn], v[dn + rt - p], j, i};
-  k.j = j;
-  k.i = i;
-  k.bu = (c.bcx + m.off)[p];
-  k.bv = (c.bcy + m.off)[p];
-  k.na0 = na[p];
-  k.nae = na[rt];
-  k.nan_ = na[up];
-  if (CROSS) {
-    const T *nb = c.Nb + m.off;
-    k.nb0 = nb[p];
-    k.nbs = nb[dn];
-    k.nbw = nb[lf];
-  } else {
-    k.nb0 = (c.Ncx + m.off)[p];
-    k.nbw = (c.Ncy + m.off)[p];
-  }
-}
