@@ -25,7 +25,8 @@ The line also carries:
                 HIP events on the library stream, over the members each
                 launch processed;
   roofline_smoother
-                the same for one fine-level smoother sweep (k_smooth_fused);
+                the same for one fine-level smoother sweep with the
+                restriction of its residual (k_fine_down);
   cpu_baseline  the CPU oracle (FP64, banded-LU linear solves) on bounded
                 samples: the smallest ensemble member on one thread (value),
                 the dome and the marine channel on one thread and on every
@@ -52,7 +53,8 @@ sys.path.insert(0, os.path.join(ROOT, "imau-ice_amd"))
 
 HBM_PEAK_GBS = 8000.0
 MFMA_BF16_PEAK_TFLOPS = 2500.0   # MI355X dense BF16 matrix-core peak
-# one fine-level smoother sweep (one k_smooth_fused launch): read u, v,
+# one fine-level smoother sweep (one k_fine_down launch, which also restricts
+# the residual, not counted here): read u, v,
 # N_a, N_b, beta_eff_cx, beta_eff_cy and the two right-hand sides, write u, v
 # (10 words per cell, 4 bytes each in the mixed mode, 8 in FP64) plus the two
 # row-type bytes
@@ -76,7 +78,7 @@ def VISC_BYTES_PER_CELL(nz, word):
 # for the headline's FP32 viscosity; other precisions are not measured.
 # Re-measure after changing either kernel.
 VISC_TRAFFIC_BYTES_PER_CELL = {"mixed_visc": 309.7}
-SWEEP_TRAFFIC_BYTES_PER_CELL = {"mixed_visc": 45.2}
+SWEEP_TRAFFIC_BYTES_PER_CELL = {}  # not measured for k_fine_down
 METHODS = {
     "learned": dict(precision="mixed_visc", mg_levels=0, picard_relax_max=0.0, ksp_type=1, anderson_m=3, learned=True,
                     text="learned warm start (BF16 conv net on the matrix cores, viscosity passes), then GCR in FP64 "
@@ -344,7 +346,7 @@ def main():
     vk = "k_visc" if visc_tile == 0 else "k_visc_march (%d rows)" % visc_tile
     roof_visc = roof("visc", "k_strain + %s (strain rates, 3D viscosity, N, F2: once per Picard iteration)" % vk,
                      VISC_BYTES_PER_CELL(nz, 4 if meth["precision"] == "mixed_visc" else 8), visc_traffic)
-    roof_sweep = roof("smoother", "k_smooth_fused (one fine-level smoother sweep)" if meth["mg_levels"] == 0
+    roof_sweep = roof("smoother", "k_fine_down (one fine-level smoother sweep and the restriction)" if meth["mg_levels"] == 0
                       else "k_prec_tile (one tile Gauss-Seidel application)",
                       SWEEP_WORDS_PER_CELL * word + SWEEP_BYTES_EXTRA, sweep_traffic if meth["mg_levels"] == 0 else None)
 
