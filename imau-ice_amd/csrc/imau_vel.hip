@@ -884,6 +884,12 @@ void reserve_buffers(imau_ctx *c, imau_problem *P, const imau_cfg *cfg) {
   if (P->pool->stream() != c->s) HIPCHK(hipDeviceSynchronize());
 }
 
+// before a call through another context than the problem's own touches its
+// state: what that one has queued (reset_state does not wait) comes first
+void after_owner(imau_ctx *c, const imau_problem *P) {
+  if (P->pool->stream() != c->s) HIPCHK(hipDeviceSynchronize());
+}
+
 // ISMIP-HOM E reads its slip columns from the 51-line Arolla file
 // (src/basal_conditions_and_sliding_module.f90:1372-1389)
 void check_ismip_e(const imau_problem *P, const imau_cfg *cfg) {
@@ -2876,9 +2882,13 @@ int imau_net_warm_start(imau_ctx *ctx, imau_problem *P, const imau_cfg *cfg, con
   const KP kp = make_kp(cfg);
   const imau::Launch L{ctx->s, (int)P->tiles.size(), P->mem_d.p, P->tiles_d.p};
   const size_t fb = P->ngrids * sizeof(int);
+  after_owner(ctx, P);
   ctx->st.h2d(ctx->s, P->act_lin.p, fb, P->sheet_any.data(), fb, 1);
   imau::net_warm(L, kp, P->F, plan->poff.p, out, P->act_lin.p);
   HIPCHK(hipGetLastError());
+  // complete on return: the problem's next solve may run on another context's
+  // stream, and the caller may free `out`
+  HIPCHK(hipStreamSynchronize(ctx->s));
   return IMAU_OK;
   ABI_CATCH(ctx)
 }

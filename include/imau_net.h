@@ -17,8 +17,8 @@
  * packed one after the other (imau_net_plan_pixels gives the level's total).
  * BF16 values are passed as uint16_t.  Convolution weights are FP32 or BF16
  * [tap][cout][cin], tap = (dr + 1) * 3 + (dc + 1); pixels outside an image
- * read as zero.  Every call is asynchronous on the context's stream;
- * imau_net_sync waits for it.  All return IMAU_OK or a negative status
+ * read as zero.  Every call but imau_net_warm_start is asynchronous on the
+ * context's stream; imau_net_sync waits for it.  All return IMAU_OK or a negative status
  * (imau_vel_last_error has the text).
  */
 #ifndef IMAU_NET_H
@@ -89,7 +89,8 @@ int imau_net_features(imau_ctx *ctx, imau_problem *P, const imau_cfg *cfg, const
  * [pix][2] asinh(u_a / 10 m/yr), asinh(v_a / 10 m/yr) and weights [pix] (1 on ice) */
 int imau_net_targets(imau_ctx *ctx, imau_problem *P, const imau_net_plan *plan, float *target, float *weight);
 /* overwrite the velocities of every member with grounded ice by the network
- * output (FP32 [pix][2], same scale as the targets) */
+ * output (FP32 [pix][2], same scale as the targets).  Complete on return: the
+ * problem may then be solved through any context, and `out` may go. */
 int imau_net_warm_start(imau_ctx *ctx, imau_problem *P, const imau_cfg *cfg, const imau_net_plan *plan,
                         const float *out);
 int imau_net_sync(imau_ctx *ctx);

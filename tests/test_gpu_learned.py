@@ -73,8 +73,8 @@ def test_features_targets_and_warm_mapping_match_oracle(env):
     rng = np.random.default_rng(0)
     o = rng.normal(scale=3.0, size=io.plan.npix[0] * 2).astype(np.float32)
     L = learned._bind(ctx.L)
-    ctx._check(L.imau_net_warm_start(ctx.h, prob.h, __import__("ctypes").byref(cfg), io.plan.h,
-                                     learned._ptr(torch.from_numpy(o).to("cuda"))))
+    o_d = torch.from_numpy(o).to("cuda")
+    ctx._check(L.imau_net_warm_start(ctx.h, prob.h, __import__("ctypes").byref(cfg), io.plan.h, learned._ptr(o_d)))
     out = prob.download()
     k = 0
     for (g, _), st in zip(mem, out):
@@ -85,6 +85,38 @@ def test_features_targets_and_warm_mapping_match_oracle(env):
         k += n
     net.release(io.plan)
     io.plan.close()
+    prob.close()
+
+
+def test_warm_start_from_another_context(env):
+    """The network in one context and the problem in another give what one
+    context gives, bit for bit, also when the network's stream still has work
+    in front of the warm start (passes over a larger plan, a few ms)."""
+    learned, solver, tw, ctx = env
+    import torch
+    cfg = tw.solver_config()
+    mem = members(learned, [4_500_000, 4_500_001], 97)
+    prob, _ = problem(solver, tw, ctx, cfg, mem)
+    with solver.Context() as other:
+        nets = [learned.Net(c, seed=0) for c in (ctx, other)]
+        out = []
+        for net in nets:
+            plan = learned.Plan(net.ctx, rows=[512] * 4, cols=[512] * 4)
+            x = torch.zeros(plan.npix[0] * learned.NFEAT, dtype=torch.int16, device="cuda")
+            ws = learned.WarmStartSolver(net.ctx, prob, net=net)
+            torch.cuda.synchronize()
+            prob.reset_state()
+            for _ in range(10):
+                net.forward(plan, x)
+            its, _ = ws.solve(cfg)
+            out.append((its, [(o["u_vav_cx"].copy(), o["v_vav_cy"].copy()) for o in prob.download()]))
+            net.sync()
+            ws.close()
+            net.release(plan)
+            plan.close()
+    assert out[0][0] == out[1][0]
+    for (ua, va), (ub, vb) in zip(out[0][1], out[1][1]):
+        assert np.array_equal(ua, ub) and np.array_equal(va, vb)
     prob.close()
 
 
