@@ -2581,6 +2581,7 @@ int imau_vel_problem_thickness(imau_ctx *ctx, imau_problem *P, int32_t g, const 
   hipStream_t s = ctx->s;
   const size_t na = (size_t)nx * ny, d8 = sizeof(double), i4 = sizeof(int32_t);
   // the member's slabs, device to device: the solved velocities stay on the GPU
+  after_owner(ctx, P);
   HIPCHK(hipMemcpyAsync((void *)D.in.Hi, P->F.Hi + pm.off, na * d8, hipMemcpyDeviceToDevice, s));
   HIPCHK(hipMemcpyAsync((void *)D.in.Hb, P->F.Hb + pm.off, na * d8, hipMemcpyDeviceToDevice, s));
   HIPCHK(hipMemcpyAsync((void *)D.in.SL, P->F.SL + pm.off, na * d8, hipMemcpyDeviceToDevice, s));

@@ -1,14 +1,15 @@
 """Kept device blocks and pinned staging of the host-array calls: what a call
 returns does not depend on the calls before it (kept blocks come back zeroed),
 on the size of its arrays against the staging buffers (2 MiB each), on another
-thread's context, or on whether the context is still open when a problem goes."""
+thread's context, on which context a problem's thickness update goes through, or
+on whether the context is still open when a problem goes."""
 import threading
 
 import numpy as np
 import pytest
 
 from imau_vel import config, geometry
-from imau_vel.state import Grid, ProducerState
+from imau_vel.state import Grid, ProducerState, ThicknessState
 
 pytestmark = pytest.mark.gpu
 
@@ -108,3 +109,40 @@ def test_problem_outlives_its_context():
     second.close()
     for f in ("u_vav_cx", "v_vav_cy", "visc_eff_3D_a", "u_3D_a"):
         np.testing.assert_array_equal(st[f], ref[f], err_msg=f)
+
+
+def test_thickness_through_another_context():
+    """reset_state does not wait; a thickness update through a second context
+    still sees the restored velocities, also when the problem's own stream has
+    work in front of the copies (network passes, a few ms)."""
+    import torch
+    from imau_vel import learned, solver
+    g, cfg, st = geometry.dome()
+    config.set_config(cfg, DIVA_visc_it_nit=3)
+    with solver.Context() as first, solver.Context() as second:
+        prob = first.problem([g], cfg, [st])
+        net = learned.Net(first, seed=0)
+        plan = learned.Plan(first, rows=[512] * 4, cols=[512] * 4)
+        x = torch.zeros(plan.npix[0] * learned.NFEAT, dtype=torch.int16, device="cuda")
+        torch.cuda.synchronize()
+        tcfg, out = config.thickness_config(), []
+        for ctx in (first, second):
+            prob.ctx = first
+            prob.solve(cfg)
+            for _ in range(10):
+                net.forward(plan, x)
+            prob.reset_state()
+            prob.ctx = ctx
+            ts = ThicknessState(g)
+            for f in ("Hi_a", "Hb_a", "SL_a", "mask_ice_a", "mask_shelf_a", "mask_ocean_a"):
+                ts[f] = st[f]
+            ts["SMB_year"], ts["float_margin_frac_a"] = 0.3, 1.0
+            prob.thickness(0, tcfg, ts, 5.0)
+            out.append(ts["dHi_dt_a"].copy())
+        net.sync()
+        net.release(plan)
+        plan.close()
+        prob.close()
+    np.testing.assert_array_equal(out[0], out[1])
+    # no velocity: the surface mass balance alone, away from the margin and the cleared boundary rows
+    np.testing.assert_allclose(out[0][10:-10, 10:-10], 0.3, rtol=1e-9)
