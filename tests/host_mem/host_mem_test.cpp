@@ -1,0 +1,94 @@
+// Checks of csrc/host_mem.h on the CPU (hip/hip_runtime.h beside this file
+// stands in for the runtime).  argv[1] names the check; 0 on success.
+#include <cstdio>
+#include <random>
+#include <thread>
+
+#include "host_mem.h"
+
+#define CHECK(x)                                                        \
+  do {                                                                  \
+    if (!(x)) {                                                         \
+      std::printf("line %d: %s\n", __LINE__, #x);                       \
+      return 1;                                                         \
+    }                                                                   \
+  } while (0)
+
+namespace {
+
+using Bytes = std::vector<unsigned char>;
+Bytes noise(size_t n, unsigned seed) {
+  std::mt19937 g(seed);
+  Bytes b(n);
+  for (auto &x : b) x = (unsigned char)g();
+  return b;
+}
+
+// rows of `row` bytes up to a device array of that pitch and down again
+bool round_trip(Stager &st, hipStream_t s, size_t row, size_t rows, size_t pitch, unsigned seed) {
+  const Bytes a = noise(row * rows, seed);
+  Bytes b(row * rows, 1), src = a;
+  Bytes dev(pitch * rows);
+  st.h2d(s, dev.data(), pitch, src.data(), row, rows);
+  std::fill(src.begin(), src.end(), 0);  // read when h2d returns
+  st.d2h(s, b.data(), dev.data(), pitch, row, rows);
+  st.flush(s);
+  return a == b;
+}
+
+int ring() {
+  hipStream_t s;
+  hipStreamCreate(&s);
+  Stager st;
+  st.flush(s);  // nothing yet
+  constexpr size_t S = Stager::kStage;
+  unsigned seed = 1;
+  for (size_t n : {(size_t)1, (size_t)255, (size_t)256, (size_t)257, S / 2 - 1, S / 2, S / 2 + 1, S, S + 8,
+                   S * Stager::kSlots, S * Stager::kSlots + 3, 3 * S * Stager::kSlots + 11})
+    CHECK(round_trip(st, s, n, 1, n, seed++));
+  // pitched: rows of a piece, rows longer than half a buffer
+  for (size_t row : {(size_t)8, (size_t)1000, S / 3, S / 2, S / 2 + 1, S + 40})
+    for (size_t rows : {(size_t)1, (size_t)2, (size_t)7}) CHECK(round_trip(st, s, row, rows, row + 24, seed++));
+  CHECK(round_trip(st, s, 24, 200000, 32, seed++));
+  CHECK(round_trip(st, s, 0, 5, 8, seed++));
+  // a later download of the same array wins
+  Bytes d1 = noise(5000, 90), d2 = noise(5000, 91), out(5000);
+  st.d2h(s, out.data(), d1.data(), 5000, 5000, 1);
+  st.d2h(s, out.data(), d2.data(), 5000, 5000, 1);
+  st.flush(s);
+  CHECK(out == d2);
+  return 0;
+}
+
+// after an error nothing more is written to the arrays of the call, and the
+// ring goes on
+int drop() {
+  hipStream_t s;
+  hipStreamCreate(&s);
+  Stager st;
+  const Bytes dev = noise(3 * Stager::kStage, 5);
+  Bytes out(dev.size(), 7);
+  st.d2h(s, out.data(), dev.data(), dev.size(), dev.size(), 1);
+  const Bytes seen = out;
+  bool threw = false;
+  try {
+    fake::st().fail_copies = 1;
+    st.d2h(s, out.data(), dev.data(), 100, 100, 1);
+  } catch (const Err &) {
+    threw = true;
+  }
+  CHECK(threw);
+  st.drop(s);
+  for (unsigned k = 0; k < 20; ++k) CHECK(round_trip(st, s, Stager::kStage, 1, Stager::kStage, k));
+  CHECK(out == seen);
+  return 0;
+}
+
+}  // namespace
+
+int main(int, char **argv) {
+  const std::string w = argv[1];
+  if (w == "ring") return ring();
+  if (w == "drop") return drop();
+  return 2;
+}
