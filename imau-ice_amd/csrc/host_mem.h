@@ -12,6 +12,7 @@
 #include <memory>
 #include <mutex>
 #include <string>
+#include <thread>
 #include <vector>
 
 #include "../../include/imau_vel.h"
@@ -175,6 +176,9 @@ void h2d(hipStream_t s, void *dst, const void *src, size_t bytes) {
 // its copy: the 66 MB of the producers at 281 x 281 x 15 cells took 85 ms, now
 // 4 ms.  h2d() has read its source when it returns; what d2h() asks for is in
 // the caller's arrays after flush().
+// Several threads may be inside calls on one context: the ring is locked for one
+// piece at a time, a flush completes the downloads of all of them (none has
+// returned, so their arrays are there), and an error drops its own thread's only.
 class Stager {
  public:
   static constexpr size_t kStage = (size_t)2 << 20;
@@ -198,27 +202,25 @@ class Stager {
     flush(s);
   }
   void flush(hipStream_t s) {
+    std::lock_guard<std::mutex> lock(mu_);
     if (!slot_[0].p) return;
     rotate(s);
     for (int k = 0; k < kSlots; ++k) reclaim((cur_ + k) % kSlots);  // oldest first
   }
-  // forget downloads that an error left unfinished (their arrays may be gone)
-  void drop(hipStream_t s) {
-    bool any = false;
-    for (const Slot &h : slot_) any = any || !h.out.empty();
-    if (!any) return;
-    (void)hipStreamSynchronize(s);
-    for (Slot &h : slot_) {
-      h.out.clear();
-      h.used = 0;
-      h.busy = false;
-    }
+  // forget this thread's downloads that an error left unfinished: their arrays
+  // may be gone.  What is in flight to the ring's own buffers may go on.
+  void drop() {
+    std::lock_guard<std::mutex> lock(mu_);
+    const std::thread::id me = std::this_thread::get_id();
+    for (Slot &h : slot_)
+      h.out.erase(std::remove_if(h.out.begin(), h.out.end(), [&](const Out &o) { return o.by == me; }), h.out.end());
   }
 
  private:
   struct Out {
     size_t at, bytes;
     char *dst;
+    std::thread::id by;
   };
   struct Slot {
     char *p = nullptr;
@@ -229,7 +231,16 @@ class Stager {
   };
   Slot slot_[kSlots];
   int cur_ = 0;
+  std::mutex mu_;
 
+  // with the lock held: create, reclaim, rotate, take
+  void create() {
+    if (slot_[kSlots - 1].ev) return;
+    for (Slot &h : slot_) {
+      if (!h.p) HIPCHK(hipHostMalloc((void **)&h.p, kStage, hipHostMallocDefault));
+      if (!h.ev) HIPCHK(hipEventCreateWithFlags(&h.ev, hipEventDisableTiming));
+    }
+  }
   void reclaim(int b) {
     Slot &h = slot_[b];
     if (h.busy) HIPCHK(hipEventSynchronize(h.ev));
@@ -257,10 +268,6 @@ class Stager {
   }
   void pieces(hipStream_t s, char *dev, size_t pitch, char *host, size_t row, size_t rows, bool up) {
     if (!row || !rows) return;
-    for (Slot &h : slot_) {
-      if (!h.p) HIPCHK(hipHostMalloc((void **)&h.p, kStage, hipHostMallocDefault));
-      if (!h.ev) HIPCHK(hipEventCreateWithFlags(&h.ev, hipEventDisableTiming));
-    }
     if (pitch == row) {  // one long row
       row *= rows;
       pitch = row;
@@ -280,6 +287,8 @@ class Stager {
   }
   void piece(hipStream_t s, char *dev, size_t pitch, char *host, size_t row, size_t rows, bool up) {
     const size_t bytes = row * rows;
+    std::lock_guard<std::mutex> lock(mu_);
+    create();
     char *p = take(s, bytes);
     if (up) std::memcpy(p, host, bytes);
     if (rows == 1)
@@ -290,7 +299,7 @@ class Stager {
       HIPCHK(hipMemcpy2DAsync(p, row, dev, pitch, row, rows, hipMemcpyDeviceToHost, s));
     if (!up) {
       Slot &h = slot_[cur_];
-      h.out.push_back(Out{(size_t)(p - h.p), bytes, host});
+      h.out.push_back(Out{(size_t)(p - h.p), bytes, host, std::this_thread::get_id()});
     }
   }
 };

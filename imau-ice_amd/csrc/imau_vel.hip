@@ -711,12 +711,12 @@ void upload(imau_ctx *c, imau_problem *P, const imau_cfg *cfg, const imau_ice_io
 #define ABI_CATCH(ctx)                                        \
   }                                                           \
   catch (const Err &e) {                                      \
-    if (ctx) (ctx)->st.drop((ctx)->s);                        \
+    if (ctx) (ctx)->st.drop();                                \
     if (ctx) (ctx)->err = e.msg; else g_init_err = e.msg;     \
     return e.code;                                            \
   }                                                           \
   catch (const std::exception &e) {                           \
-    if (ctx) (ctx)->st.drop((ctx)->s);                        \
+    if (ctx) (ctx)->st.drop();                                \
     if (ctx) (ctx)->err = e.what(); else g_init_err = e.what(); \
     return IMAU_ERR_DEVICE;                                   \
   }

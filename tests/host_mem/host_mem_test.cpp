@@ -78,9 +78,48 @@ int drop() {
     threw = true;
   }
   CHECK(threw);
-  st.drop(s);
+  st.drop();
   for (unsigned k = 0; k < 20; ++k) CHECK(round_trip(st, s, Stager::kStage, 1, Stager::kStage, k));
   CHECK(out == seen);
+  return 0;
+}
+
+// a call of another thread on the same context that ends on an error does not
+// take this one's pending downloads with it
+int drop_of_another_thread() {
+  hipStream_t s;
+  hipStreamCreate(&s);
+  Stager st;
+  const Bytes dev = noise(100000, 5), dev2 = noise(70000, 6);
+  Bytes out(dev.size()), out2(dev2.size(), 7);
+  st.d2h(s, out.data(), dev.data(), dev.size(), dev.size(), 1);
+  std::thread([&] {
+    st.d2h(s, out2.data(), dev2.data(), dev2.size(), dev2.size(), 1);
+    st.drop();
+  }).join();
+  st.flush(s);
+  CHECK(out == dev);
+  CHECK(out2 == Bytes(dev2.size(), 7));
+  return 0;
+}
+
+// calls of several threads on one context
+int threads() {
+  hipStream_t s;
+  hipStreamCreate(&s);
+  Stager st;
+  std::atomic<int> bad{0};
+  std::vector<std::thread> ts;
+  for (unsigned q = 0; q < 4; ++q)
+    ts.emplace_back([&, q] {
+      std::mt19937 g(q);
+      for (unsigned k = 0; k < 60; ++k) {
+        const size_t row = 1 + g() % 50000, rows = 1 + g() % 20;
+        if (!round_trip(st, s, row, rows, row + g() % 2 * 8, 100 * q + k)) ++bad;
+      }
+    });
+  for (auto &t : ts) t.join();
+  CHECK(bad == 0);
   return 0;
 }
 
@@ -90,5 +129,7 @@ int main(int, char **argv) {
   const std::string w = argv[1];
   if (w == "ring") return ring();
   if (w == "drop") return drop();
+  if (w == "drop_of_another_thread") return drop_of_another_thread();
+  if (w == "threads") return threads();
   return 2;
 }

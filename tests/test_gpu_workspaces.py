@@ -1,7 +1,7 @@
 """Kept device blocks and pinned staging of the host-array calls: what a call
 returns does not depend on the calls before it (kept blocks come back zeroed),
 on the size of its arrays against the staging buffers (2 MiB each), on another
-thread's context, on which context a problem's thickness update goes through, or
+thread's context or calls, on which context a problem's thickness update goes through, or
 on whether the context is still open when a problem goes."""
 import threading
 
@@ -81,6 +81,49 @@ def test_contexts_of_two_threads():
     assert not errs, errs
     for q in range(2):
         same(got[q], ref[q])
+
+
+def test_two_threads_in_one_context():
+    """Host-array calls of two threads on the same context, bit for bit."""
+    from imau_vel import solver
+    g = Grid(281, 283, 8e3)
+    rng = np.random.default_rng(7)
+    ts, ps = ThicknessState(g), ProducerState(g, 15)
+    ts["Hi_a"] = rng.uniform(500.0, 900.0, (g.ny, g.nx))
+    ts["u_vav_cx"] = rng.uniform(-150.0, 150.0, (g.ny, g.nx - 1))
+    ts["v_vav_cy"] = rng.uniform(-150.0, 150.0, (g.ny - 1, g.nx))
+    ts["mask_ice_a"], ts["float_margin_frac_a"] = 1, 1.0
+    for f in ("mask_ice_a", "mask_sheet_a"):
+        ps[f] = 1
+    ps["Ti_a"] = rng.uniform(240.0, 262.0, (15, g.ny, g.nx))
+    tcfg, pcfg = config.thickness_config(choice_ice_integration_method="explicit"), config.producer_config()
+
+    def thickness(ctx):
+        out = ts.copy()
+        ctx.thickness_update(g, tcfg, out, 2.0)
+        return [out[f].copy() for f in ("dHi_dt_a", "Hi_tplusdt_a", "Qx_cx", "Qy_cy")]
+
+    def rheology(ctx):
+        ctx.calc_ice_rheology(g, pcfg, ps)
+        return [ps[f].copy() for f in ("A_flow_3D_a", "A_flow_3D_cx", "A_flow_3D_cy", "A_flow_vav_a", "A_flow_vav_cy")]
+
+    calls, errs, bad = (thickness, rheology), [], []
+    with solver.Context() as ctx:
+        ref = [f(ctx) for f in calls]
+
+        def work(q):
+            try:
+                for _ in range(20):
+                    if not all(np.array_equal(a, b) for a, b in zip(calls[q](ctx), ref[q])):
+                        bad.append(q)
+            except Exception as e:
+                errs.append(e)
+        threads = [threading.Thread(target=work, args=(q,)) for q in range(2)]
+        for t in threads:
+            t.start()
+        for t in threads:
+            t.join()
+    assert not errs and not bad, (errs, bad)
 
 
 def test_problem_outlives_its_context():

@@ -19,7 +19,7 @@ def program(tmp_path_factory):
     return exe
 
 
-@pytest.mark.parametrize("check", ["ring", "drop"])
+@pytest.mark.parametrize("check", ["ring", "drop", "drop_of_another_thread", "threads"])
 def test_host_mem(program, check):
     r = subprocess.run([program, check], stdout=subprocess.PIPE, text=True, timeout=120)
     assert r.returncode == 0, r.stdout
