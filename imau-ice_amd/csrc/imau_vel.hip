@@ -792,7 +792,7 @@ int imau_vel_init(const imau_grid *grid, const imau_cfg *cfg, imau_ctx **out) {
   ctx = new imau_ctx();
   HIPCHK(hipGetDevice(&ctx->device));
   HIPCHK(hipStreamCreateWithFlags(&ctx->s, hipStreamNonBlocking));
-  ctx->pool = std::make_shared<DevPool>(ctx->s);
+  ctx->pool = Pool{std::make_shared<DevPool>(ctx->s)};
   ctx->scratch = scratch_address(ctx->device);
   *out = ctx;
   return IMAU_OK;
@@ -833,15 +833,26 @@ int imau_vel_kernel_timing(imau_ctx *ctx, int32_t what, int64_t *launches, doubl
   return IMAU_OK;
 }
 
-int imau_vel_problem_create(imau_ctx *ctx, int32_t ngrids, const imau_grid *grids, const imau_cfg *cfg,
-                            const imau_ice_io *ios, imau_problem **prob) {
+int imau_vel_keep_memory(imau_ctx *ctx, int64_t bytes, int64_t *kept) {
+  ABI_TRY
+  if (!ctx) fail(IMAU_ERR_ARG, "NULL argument");
+  if (bytes >= 0) ctx->pool->set_limit((size_t)bytes);
+  if (kept) *kept = (int64_t)ctx->pool->kept();
+  return IMAU_OK;
+  ABI_CATCH(ctx)
+}
+
+// pool: the context's, for a problem that lives for one call on host arrays; its
+// given_back() handle for one that the caller owns
+static int problem_create(imau_ctx *ctx, const Pool &pool, int32_t ngrids, const imau_grid *grids, const imau_cfg *cfg,
+                          const imau_ice_io *ios, imau_problem **prob) {
   imau_problem *P = nullptr;
   ABI_TRY
   if (!ctx || !grids || !ios || !prob) fail(IMAU_ERR_ARG, "NULL argument");
   if (ngrids < 1) fail(IMAU_ERR_ARG, "ngrids=%d", ngrids);
   check_cfg(cfg);
   P = new imau_problem();
-  P->pool = ctx->pool;
+  P->pool = pool;
   P->ngrids = ngrids;
   P->nz = cfg->nz;
   long long off = 0, offx = 0, offy = 0;
@@ -943,9 +954,14 @@ int imau_vel_problem_create(imau_ctx *ctx, int32_t ngrids, const imau_grid *grid
   }
 }
 
+int imau_vel_problem_create(imau_ctx *ctx, int32_t ngrids, const imau_grid *grids, const imau_cfg *cfg,
+                            const imau_ice_io *ios, imau_problem **prob) {
+  return problem_create(ctx, ctx ? ctx->pool.given_back() : Pool{}, ngrids, grids, cfg, ios, prob);
+}
+
 void imau_vel_problem_destroy(imau_problem *P) {
   if (!P) return;
-  (void)hipDeviceSynchronize();  // its memory may be handed out again at once
+  (void)hipDeviceSynchronize();  // its memory goes at once
   delete P;
 }
 
@@ -1941,7 +1957,7 @@ static int solve_convenience(imau_ctx *ctx, int ngrids, const imau_grid *grids, 
                              int kinds) {
   if (!ctx) return IMAU_ERR_ARG;
   imau_problem *P = nullptr;
-  int rc = imau_vel_problem_create(ctx, ngrids, grids, cfg, ios, &P);
+  int rc = problem_create(ctx, ctx->pool, ngrids, grids, cfg, ios, &P);
   if (rc) return rc;
   rc = solve_kind(ctx, P, cfg, kinds);
   if (!rc) rc = imau_vel_problem_download(ctx, P, ios);
@@ -1972,7 +1988,7 @@ int imau_vel_nonlinear_residual(imau_ctx *ctx, const imau_grid *grid, const imau
   } release{P};
   ABI_TRY
   if (!ctx || !grid || !cfg || !io || !residual) fail(IMAU_ERR_ARG, "NULL argument");
-  int rc = imau_vel_problem_create(ctx, 1, grid, cfg, io, &P);
+  int rc = problem_create(ctx, ctx->pool, 1, grid, cfg, io, &P);
   if (rc) return rc;
   const bool diva = cfg->choice_ice_dynamics == IMAU_DYN_DIVA;
   Solver S(ctx, P, cfg);
@@ -2416,7 +2432,7 @@ int imau_net_plan_create(imau_ctx *ctx, int32_t nimg, const int32_t *rows, const
   for (int g = 0; g < nimg; ++g)
     if (rows[g] < 1 || cols[g] < 1) fail(IMAU_ERR_ARG, "image %d is %d x %d", g, rows[g], cols[g]);
   N = new imau_net_plan();
-  net_plan_build(ctx->pool, ctx->s, N, nimg, rows, cols);
+  net_plan_build(ctx->pool.given_back(), ctx->s, N, nimg, rows, cols);
   HIPCHK(hipDeviceSynchronize());  // the plan may be used on another stream's data
   *plan = N;
   return IMAU_OK;
@@ -2439,7 +2455,7 @@ int imau_net_plan_for_problem(imau_ctx *ctx, const imau_problem *P, imau_net_pla
 
 void imau_net_plan_destroy(imau_net_plan *plan) {
   if (!plan) return;
-  (void)hipDeviceSynchronize();  // its memory may be handed out again at once
+  (void)hipDeviceSynchronize();  // its memory goes at once
   delete plan;
 }
 
@@ -2892,7 +2908,7 @@ int run_loop(imau_ctx *ctx, const imau_grid *grid, const imau_cfg *cfg, const im
   imau_cfg vcfg = *cfg;
   if (dyn == IMAU_DYN_NONE) vcfg.choice_ice_dynamics = IMAU_DYN_SIA;  // the problem only carries the geometry
   imau_problem *P = nullptr;
-  int rc = imau_vel_problem_create(ctx, 1, grid, &vcfg, io, &P);
+  int rc = problem_create(ctx, ctx->pool, 1, grid, &vcfg, io, &P);
   if (rc) return rc;
   struct Release {
     imau_problem *&p;

@@ -412,6 +412,13 @@ MODULE imau_vel_bindings
       IMPORT :: C_PTR
       TYPE(C_PTR), VALUE :: ctx
     END SUBROUTINE
+    FUNCTION imau_vel_keep_memory(ctx, bytes, kept) BIND(C, name='imau_vel_keep_memory') RESULT(rc)
+      IMPORT :: C_INT, C_INT64_T, C_PTR
+      TYPE(C_PTR), VALUE :: ctx
+      INTEGER(C_INT64_T), VALUE :: bytes
+      INTEGER(C_INT64_T), INTENT(OUT) :: kept
+      INTEGER(C_INT) :: rc
+    END FUNCTION
     FUNCTION imau_vel_last_error(ctx) BIND(C, name='imau_vel_last_error') RESULT(msg)
       IMPORT :: C_PTR
       TYPE(C_PTR), VALUE :: ctx

@@ -24,6 +24,7 @@ EXPORTED = (
     "imau_vel_problem_download", "imau_vel_problem_destroy", "imau_vel_solve_diva_batch",
     "imau_vel_kernel_timing", "imau_vel_problem_stats", "imau_vel_problem_residual_noalloc",
     "imau_vel_problem_restarts", "imau_vel_problem_thickness", "imau_vel_problem_autotune", "imau_vel_problem_set_tile_rows",
+    "imau_vel_keep_memory",
 )
 # the ice-thickness update that consumes the velocities
 THICKNESS_EXPORTED = ("imau_thickness_default_config", "imau_thickness_update", "imau_critical_timestep_adv")
@@ -70,6 +71,7 @@ def load_library(path: str = LIB_PATH):
     L.imau_vel_problem_destroy.restype = None
     L.imau_vel_solve_diva_batch.argtypes = [vp, ctypes.c_int32, P(ImauGrid), P(ImauCfg), P(ImauIceIO)]
     L.imau_vel_kernel_timing.argtypes = [vp, ctypes.c_int32, P(ctypes.c_int64), P(ctypes.c_double), P(ctypes.c_int64)]
+    L.imau_vel_keep_memory.argtypes = [vp, ctypes.c_int64, P(ctypes.c_int64)]
     L.imau_vel_problem_stats.argtypes = [vp, vp, P(ctypes.c_int32), P(ctypes.c_double)]
     L.imau_vel_problem_restarts.argtypes = [vp, vp, P(ctypes.c_int32)]
     L.imau_vel_problem_autotune.argtypes = [vp, vp, P(ImauCfg), P(ctypes.c_int32)]
@@ -224,6 +226,14 @@ class Context:
         n, ms, cells = ctypes.c_int64(), ctypes.c_double(), ctypes.c_int64()
         self._check(self.L.imau_vel_kernel_timing(self.h, code, ctypes.byref(n), ctypes.byref(ms), ctypes.byref(cells)))
         return n.value, ms.value, cells.value
+
+    def keep_memory(self, nbytes=-1):
+        """Bytes of device memory that the host-array calls of this context have
+        left for the next one.  nbytes >= 0 first sets the most that is kept
+        (4 GiB at the start; 0 gives everything back to the driver)."""
+        kept = ctypes.c_int64()
+        self._check(self.L.imau_vel_keep_memory(self.h, nbytes, ctypes.byref(kept)))
+        return kept.value
 
     def problem(self, grids, cfg, states):
         return Problem(self, grids, cfg, states)

@@ -294,6 +294,18 @@ const char *imau_vel_last_error(const imau_ctx *ctx);
 enum { IMAU_TIME_OFF = 0, IMAU_TIME_SMOOTHER = 1, IMAU_TIME_VISC = 2 };
 int  imau_vel_kernel_timing(imau_ctx *ctx, int32_t what, int64_t *launches, double *ms, int64_t *cells);
 
+/* Device memory (no reference counterpart).  The calls that take host arrays
+ * (imau_vel_solve_*, imau_vel_nonlinear_residual, the thickness update, the
+ * producers, the time loops) keep the device buffers they have used for the
+ * context's next such call, at most 4 GiB of them.  They go back to the driver
+ * with imau_vel_finalize, when an allocation of any context in the process would
+ * fail otherwise, and with this call: at most `bytes` are kept from now on (0:
+ * all is given back and nothing kept; negative: no change).  *kept (may be NULL)
+ * receives the bytes kept now.  Other users of the GPU in the process (PyTorch)
+ * cannot ask for them.  The memory of a problem or a network plan goes back
+ * when it is destroyed. */
+int  imau_vel_keep_memory(imau_ctx *ctx, int64_t bytes, int64_t *kept);
+
 /* Fills cfg with the reference defaults (src/configuration_module.f90). */
 void imau_vel_default_config(imau_cfg *cfg);
 

@@ -123,6 +123,137 @@ int threads() {
   return 0;
 }
 
+Pool new_pool() {
+  hipStream_t s;
+  hipStreamCreate(&s);
+  return Pool{std::make_shared<DevPool>(s)};
+}
+bool zero(const DBuf<char> &b) {
+  return std::all_of(b.p, b.p + b.n, [](char c) { return c == 0; });
+}
+
+// kept blocks are handed out again, zeroed, in the order of the stream
+int reuse() {
+  const Pool pool = new_pool();
+  DBuf<char> a, b;
+  a.alloc(pool, 10000);
+  hipStreamSynchronize(pool->stream());
+  CHECK(zero(a));
+  hipMemsetAsync(a.p, 1, a.n, pool->stream());
+  const char *was = a.p;
+  a.release();
+  CHECK(pool->kept() == 12288 && fake::st().live == 12288);
+  b.alloc(pool, 13000);  // does not fit
+  CHECK(b.p != was);
+  a.alloc(pool, 9000);   // within a quarter
+  CHECK(a.p == was && pool->kept() == 0);
+  hipStreamSynchronize(pool->stream());
+  CHECK(zero(a) && zero(b));
+  return 0;
+}
+
+// at most limit() bytes are kept, the oldest go first, a limit of 0 gives all back
+int limit() {
+  const Pool pool = new_pool();
+  pool->set_limit(5 << 20);
+  DBuf<char> b[4];
+  const char *last = nullptr;
+  for (int k = 0; k < 4; ++k) b[k].alloc(pool, (size_t)(k + 1) << 20);
+  for (auto &x : b) last = x.p, x.release();  // 1 + 2 MiB, then 3, then 4: the older ones go
+  CHECK(pool->kept() == (4 << 20) && fake::st().live == (4 << 20));
+  b[0].alloc(pool, 4 << 20);
+  CHECK(b[0].p == last);
+  b[1].alloc(pool, 6 << 20);  // more than the limit: straight back
+  b[1].release();
+  CHECK(pool->kept() == 0 && fake::st().live == (4 << 20));
+  b[0].release();
+  pool->set_limit(0);
+  CHECK(pool->kept() == 0 && fake::st().live == 0);
+  b[0].alloc(pool, 100);
+  b[0].release();
+  CHECK(fake::st().live == 0);
+  return 0;
+}
+
+// what the caller owns goes back to the driver
+int given_back() {
+  const Pool pool = new_pool();
+  DBuf<char> kept, own;
+  kept.alloc(pool, 1 << 20);
+  kept.release();
+  own.alloc(pool.given_back(), 1 << 20);
+  CHECK(pool->kept() == (1 << 20) && fake::st().live == (2 << 20));
+  hipStreamSynchronize(pool->stream());
+  CHECK(zero(own));
+  own.release();
+  CHECK(pool->kept() == (1 << 20) && fake::st().live == (1 << 20));
+  return 0;
+}
+
+// when the driver has no more, every context gives back what it keeps
+int out_of_memory() {
+  const Pool mine = new_pool(), other = new_pool();
+  DBuf<char> a, b;
+  for (const Pool &p : {mine, other}) {
+    a.alloc(p, 3 << 20);
+    a.release();
+  }
+  fake::st().limit = 7 << 20;
+  b.alloc(mine, 5 << 20);
+  CHECK(mine->kept() == 0 && other->kept() == 0 && fake::st().live == (5 << 20));
+  b.release();
+  bool threw = false;
+  try {
+    a.alloc(other.given_back(), 8 << 20);
+  } catch (const Err &) {
+    threw = true;
+  }
+  CHECK(threw && fake::st().live == 0);
+  return 0;
+}
+
+// buffers that outlive the context
+int closed() {
+  Pool pool = new_pool();
+  DBuf<char> a, b;
+  a.alloc(pool, 5000);
+  b.alloc(pool, 5000);
+  a.release();
+  pool->close();
+  CHECK(pool->kept() == 0 && fake::st().live == 8192);
+  a.alloc(pool, 3000);
+  CHECK(zero(a));  // nothing to wait for
+  pool = Pool{};
+  a.release();
+  b.release();
+  CHECK(fake::st().live == 0);
+  return 0;
+}
+
+// allocations of several threads and contexts, with less memory than they want to keep
+int pool_threads() {
+  const Pool pools[2] = {new_pool(), new_pool()};
+  fake::st().limit = 24 << 20;
+  std::atomic<int> bad{0};
+  std::vector<std::thread> ts;
+  for (unsigned q = 0; q < 4; ++q)
+    ts.emplace_back([&, q] {
+      std::mt19937 g(q);
+      const Pool &pool = pools[q & 1];
+      for (int k = 0; k < 200; ++k) {
+        DBuf<char> a, b;
+        a.alloc(pool, 1 + g() % (2 << 20));
+        b.alloc(pool.given_back(), 1 + g() % (1 << 20));
+        hipStreamSynchronize(pool->stream());
+        if (!zero(a) || !zero(b)) ++bad;
+        std::fill(a.p, a.p + a.n, (char)1);
+      }
+    });
+  for (auto &t : ts) t.join();
+  CHECK(bad == 0);
+  return 0;
+}
+
 }  // namespace
 
 int main(int, char **argv) {
@@ -131,5 +262,11 @@ int main(int, char **argv) {
   if (w == "drop") return drop();
   if (w == "drop_of_another_thread") return drop_of_another_thread();
   if (w == "threads") return threads();
+  if (w == "reuse") return reuse();
+  if (w == "limit") return limit();
+  if (w == "given_back") return given_back();
+  if (w == "out_of_memory") return out_of_memory();
+  if (w == "closed") return closed();
+  if (w == "pool_threads") return pool_threads();
   return 2;
 }

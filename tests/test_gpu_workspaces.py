@@ -1,5 +1,6 @@
 """Kept device blocks and pinned staging of the host-array calls: what a call
-returns does not depend on the calls before it (kept blocks come back zeroed),
+returns does not depend on the calls before it (kept blocks come back zeroed; they
+go back to the driver on demand),
 on the size of its arrays against the staging buffers (2 MiB each), on another
 thread's context or calls, on which context a problem's thickness update goes through, or
 on whether the context is still open when a problem goes."""
@@ -124,6 +125,30 @@ def test_two_threads_in_one_context():
         for t in threads:
             t.join()
     assert not errs and not bad, (errs, bad)
+
+
+def test_device_memory_goes_back():
+    """What host-array calls keep is reported and given back on demand, and a
+    destroyed problem's memory (10 MB and more here) goes back by itself."""
+    import torch
+    from imau_vel import solver
+    with solver.Context() as ctx:
+        ref = solve(ctx, 61, 57)
+        assert ctx.keep_memory() > 0
+        assert ctx.keep_memory(0) == 0
+        same(solve(ctx, 61, 57), ref)
+        assert ctx.keep_memory() == 0
+        ctx.keep_memory(4 << 30)
+        same(solve(ctx, 61, 57), ref)
+        kept = ctx.keep_memory()
+        assert 0 < kept <= 4 << 30
+        g, cfg, st = geometry.dome(201, 203, 8e3)
+        free = torch.cuda.mem_get_info()[0]
+        prob = ctx.problem([g], cfg, [st])
+        assert torch.cuda.mem_get_info()[0] < free
+        prob.close()
+        assert torch.cuda.mem_get_info()[0] >= free - (8 << 20)    # the driver's own granularity
+        assert ctx.keep_memory() == kept
 
 
 def test_problem_outlives_its_context():

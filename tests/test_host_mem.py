@@ -19,7 +19,8 @@ def program(tmp_path_factory):
     return exe
 
 
-@pytest.mark.parametrize("check", ["ring", "drop", "drop_of_another_thread", "threads"])
+@pytest.mark.parametrize("check", ["ring", "drop", "drop_of_another_thread", "threads", "reuse", "limit",
+                                   "given_back", "out_of_memory", "closed", "pool_threads"])
 def test_host_mem(program, check):
     r = subprocess.run([program, check], stdout=subprocess.PIPE, text=True, timeout=120)
     assert r.returncode == 0, r.stdout
