@@ -45,10 +45,11 @@
 // 51; then it grows by 0.16 us a tile (109 / 46 at 637), the tiled one stays
 #define IMAU_LEVMAX 16
 #define IMAU_LEVTILES 56
-// workgroups per tile of the tiled kernel: one row per wavefront (us with one
-// and two: 28.6 / 16.7 at 51 tiles, 54 / 46 at 637, both FP64; FP32 40 / 38.5
-// at 1024, 102 / 94 at 3000)
-#define IMAU_VISC_GY (IMAU_VTI / IMAU_WG_I)
+// workgroups per tile of the tiled kernel: one row per wavefront.  DIVA, 15
+// levels, us with one and two: FP64 29.8 / 16.5 at 64 tiles, 32.8 / 24.0 at 256,
+// 53.4 / 46.0 at 637, 187 / 180 at 3072; FP32 22.7 / 14.0, 24.1 / 16.5, 30.5 /
+// 23.2, 112 / 105; with k_strain on the 64 uneven caps (15655 tiles) 567 / 563
+#define IMAU_VISC_PARTS (IMAU_VTI / IMAU_WG_I)
 
 // Workgroups are dispatched round-robin over the 8 XCDs (workgroup b on XCD
 // b % 8), each with its own L2.  Tile kernels run tile imau_xcd_tile() rather
@@ -56,7 +57,11 @@
 // tile list, so the halo rows and columns that neighbouring tiles share are
 // fetched into one L2 rather than two.  A bijection of [0, gridDim.x); per-tile
 // partial sums are stored at the tile's index, so each member's partials stay
-// contiguous.
+// contiguous.  Kernels that split a tile over several workgroups launch
+// tiles x parts workgroups in one dimension, the parts of a tile next to each
+// other, so that they stay on the tile's XCD.  A second grid dimension moves
+// part y by y * gridDim.x workgroups, to another XCD: k_strain + k_visc on the
+// 64 uneven caps took 576 us that way.
 __device__ __forceinline__ int imau_xcd_tile() {
   const int n = (int)gridDim.x, b = (int)blockIdx.x;
   const int q = n >> 3, r = n & 7, x = b & 7;

@@ -14,9 +14,16 @@
   const Member m = mem[t.g];                        \
   const int j = t.j0 + (int)threadIdx.x;
 
+// one of the `parts` workgroups of a tile
+#define TILE_SETUP_PARTS(parts)                               \
+  const int tp = imau_xcd_tile(), part = tp % (parts);        \
+  const Tile t = tiles[tp / (parts)];                         \
+  const Member m = mem[t.g];                                  \
+  const int j = t.j0 + (int)threadIdx.x;
+
 #define FOR_TILE_ROWS for (int ii = threadIdx.y; ii < IMAU_TI; ii += IMAU_WG_I)
-// with the rows of a tile dealt to gridDim.y workgroups
-#define FOR_VTILE_ROWS_Y _Pragma("unroll 1") for (int ii = threadIdx.y + IMAU_WG_I * blockIdx.y; ii < IMAU_VTI; ii += IMAU_WG_I * gridDim.y)
+// with the rows of a tile dealt to IMAU_VISC_PARTS workgroups
+#define FOR_VTILE_ROWS_PART _Pragma("unroll 1") for (int ii = threadIdx.y + IMAU_WG_I * part; ii < IMAU_VTI; ii += IMAU_WG_I * IMAU_VISC_PARTS)
 #define FOR_VTILE_ROWS _Pragma("unroll 1") for (int ii = threadIdx.y; ii < IMAU_VTI; ii += IMAU_WG_I)
 
 // ---------------------------------------------------------------------------
@@ -499,18 +506,18 @@ __global__ void __launch_bounds__(IMAU_WG) k_visc(const Member *__restrict__ mem
                                                   const KP kp, const Fields f, const T *__restrict__ visc_in,
                                                   T *__restrict__ visc_out, const T *__restrict__ B3,
                                                   const int *__restrict__ active) {
-  TILE_SETUP
+  TILE_SETUP_PARTS(IMAU_VISC_PARTS)
   if (j >= m.ny) return;
   const int nx = m.nx, ny = m.ny, nz = kp.nz;
   if (!active[t.g]) {  // finished member: keep its viscosity in the buffer that becomes current
-    FOR_VTILE_ROWS_Y {
+    FOR_VTILE_ROWS_PART {
       const int i = t.i0 + ii;
       if (i >= nx) break;
       for (int k = 0; k < nz; ++k) visc_out[p3(m, k, j, i)] = visc_in[p3(m, k, j, i)];
     }
     return;
   }
-  FOR_VTILE_ROWS_Y {
+  FOR_VTILE_ROWS_PART {
     const int i = t.i0 + ii;
     if (i >= nx) break;
     const long long p = p2(m, j, i);
@@ -592,9 +599,9 @@ __global__ void __launch_bounds__(IMAU_TJ *IMAU_LEVMAX) k_visc_lev(
     const Member *__restrict__ mem, const Tile *__restrict__ tiles, const KP kp, const Fields f,
     const T *__restrict__ visc_in, T *__restrict__ visc_out, const T *__restrict__ B3, const int *__restrict__ active) {
   __shared__ T s_eta[IMAU_LEVMAX][IMAU_TJ], s_g[DIVA ? IMAU_LEVMAX : 1][IMAU_TJ];
-  TILE_SETUP
+  TILE_SETUP_PARTS(IMAU_VTI)
   const int nx = m.nx, ny = m.ny, nz = kp.nz;
-  const int i = t.i0 + (int)blockIdx.y, k = __builtin_amdgcn_readfirstlane(threadIdx.y);
+  const int i = t.i0 + part, k = __builtin_amdgcn_readfirstlane(threadIdx.y);
   if (i >= nx) return;  // the whole workgroup
   const bool in = j < ny;
   const long long q = p3(m, k, min(j, ny - 1), i);
@@ -1798,13 +1805,13 @@ static void visc_tiles(const Launch &L, const Launch &LV, const KP &kp, const Fi
   if (kp.nz <= IMAU_LEVMAX && LV.ntiles <= IMAU_LEVTILES) {
     auto kl = diva ? (third ? k_visc_lev<true, true, T> : k_visc_lev<true, false, T>)
                    : (third ? k_visc_lev<false, true, T> : k_visc_lev<false, false, T>);
-    hipLaunchKernelGGL(kl, dim3(LV.ntiles, IMAU_VTI), dim3(IMAU_TJ, kp.nz), 0, L.s, L.mem, LV.tiles, kp, f, visc_in,
+    hipLaunchKernelGGL(kl, dim3(LV.ntiles * IMAU_VTI), dim3(IMAU_TJ, kp.nz), 0, L.s, L.mem, LV.tiles, kp, f, visc_in,
                        visc_out, B3, active);
     return;
   }
   auto kv = diva ? (third ? k_visc<true, true, T> : k_visc<true, false, T>)
                  : (third ? k_visc<false, true, T> : k_visc<false, false, T>);
-  hipLaunchKernelGGL(kv, dim3(LV.ntiles, IMAU_VISC_GY), wg(), 0, L.s, L.mem, LV.tiles, kp, f, visc_in, visc_out, B3, active);
+  hipLaunchKernelGGL(kv, dim3(LV.ntiles * IMAU_VISC_PARTS), wg(), 0, L.s, L.mem, LV.tiles, kp, f, visc_in, visc_out, B3, active);
 }
 void visc3d(const Launch &L, const Launch &LV, const KP &kp, const Fields &f, bool diva, const double *visc_in,
             double *visc_out, const int *active) {

@@ -353,15 +353,15 @@ __global__ void __launch_bounds__(IMAU_WG) k_gal0_plain(const Member *__restrict
   }
 }
 
-// level l (Fl) -> level l+1 (L), accumulated in FP64; blockIdx.y is the
-// component.  Slot k of a fine row addresses the unknown at constant offsets,
-// so its coarse slot is a constant, at the level's edges too: a slot whose
-// unknown lies outside the level holds zero (no sum ever writes another value
-// into it), and only whole fine cells past an odd edge have to be masked.  Bound
-// by load latency, so the 36 coefficients of a cell are loaded before any is
-// added; testing every coupling's bounds instead, with a straight-line path for
-// the interior beside it, serialised the loads:
-// 38-41 us, now 6.1 us (401 x 41 channel, FP64) and 7.2 us (12 caps, FP32).
+// level l (Fl) -> level l+1 (L), accumulated in FP64; two workgroups per tile,
+// one per component.  Slot k of a fine row addresses the unknown at constant
+// offsets, so its coarse slot is a constant, at the level's edges too: a slot
+// whose unknown lies outside the level holds zero (no sum ever writes another
+// value into it), and only whole fine cells past an odd edge have to be masked.
+// Bound by load latency, so the 36 coefficients of a cell are loaded before any
+// is added; testing every coupling's bounds instead, with a straight-line path
+// for the interior beside it, serialised the loads: 38-41 us, now 6.1 us (401 x
+// 41 channel, FP64) and 7.2 us (12 caps, FP32).
 template <class T, int COMP>
 __device__ __forceinline__ void galc_cell(const CLevelT<T> &Fl, const CMember &fm, const CLevelT<T> &L, int J, int I,
                                           long long pc) {
@@ -395,14 +395,17 @@ __device__ __forceinline__ void galc_cell(const CLevelT<T> &Fl, const CMember &f
 
 template <class T>
 __global__ void __launch_bounds__(IMAU_WG) k_galc(CLevelT<T> Fl, CLevelT<T> L, const int *__restrict__ active) {
-  CTILE_SETUP
+  const int tp = imau_xcd_tile(), comp = tp & 1;
+  const Tile t = L.tiles[tp >> 1];
+  const CMember cm = L.mem[t.g];
+  const int J = t.j0 + (int)threadIdx.x;
   if (J >= cm.ny || !active[t.g] || L.depth[t.g] < L.lev) return;
   const CMember fm = Fl.mem[t.g];
   FOR_TILE_ROWS {
     const int I = t.i0 + ii;
     if (I >= cm.nx) break;
     const long long pc = cp2(cm, J, I);
-    if (blockIdx.y == 0) {
+    if (comp == 0) {
       if (cvalid(cm, 0, J, I)) galc_cell<T, 0>(Fl, fm, L, J, I, pc);
     } else {
       if (cvalid(cm, 1, J, I)) galc_cell<T, 1>(Fl, fm, L, J, I, pc);
@@ -1270,7 +1273,7 @@ void setup_t(const imau::Launch &F, const KP &kp, const imau::Coef &c, const ima
   }
   for (size_t l = 1; l < P.levels.size(); ++l) {
     const CLevelT<T> Fl = view<T>(P, (int)l - 1), L = view<T>(P, (int)l);
-    hipLaunchKernelGGL(k_galc<T>, dim3(L.ntiles, 2), wg(), 0, F.s, Fl, L, act);
+    hipLaunchKernelGGL(k_galc<T>, dim3(2 * L.ntiles), wg(), 0, F.s, Fl, L, act);
   }
 }
 
