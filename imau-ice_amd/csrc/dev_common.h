@@ -40,11 +40,17 @@
 #define IMAU_MTI_CANDIDATES {0, 4, 8, 16, 32}
 #define IMAU_MNZ 15
 // small-grid viscosity kernel (one wavefront per level): most levels (the
-// wavefronts of a workgroup) and most IMAU_VTI-row tiles.  FP64 DIVA, 15
-// levels, us against the tiled kernel: 8.4 / 16.8 at 6 tiles, 14.9 / 16.7 at
-// 51; then it grows by 0.16 us a tile (109 / 46 at 637), the tiled one stays
+// wavefronts of a workgroup) and most IMAU_VTI-row tiles.  Its time goes in
+// steps of 32 tiles (one workgroup per CU); k_visc's hardly changes.  us with 64
+// and 72 tiles, by level / tiled kernel: DIVA, 15 levels, FP64 13.8 / 16.5 and
+// 18.7 / 16.9, FP32 9.6 / 14.0 and 12.9 / 14.2; n = 4, FP64 16.7 / 23.0 and 22.8 /
+// 23.4; 8 levels 8.4 / 11.1 and 10.4 / 11.0; SSA, 15 levels, FP64 5.3 / 5.6 and
+// 6.6 / 5.9, FP32 4.6 / 5.1 and 5.5 / 5.3 (3 levels: 3.6 / 3.3 at any size).  At 4
+// tiles DIVA takes 7.8 / 16.1.  SSA in FP64 with n != 3 keeps the tiled kernel
+// (7.8 / 6.0 at 64 tiles, 5.7 / 5.6 at 16): its strain rate is the same at every
+// level, so a column needs one pow(), not one per level.
 #define IMAU_LEVMAX 16
-#define IMAU_LEVTILES 56
+#define IMAU_LEVTILES 64
 // workgroups per tile of the tiled kernel: one row per wavefront.  DIVA, 15
 // levels, us with one and two: FP64 29.8 / 16.5 at 64 tiles, 32.8 / 24.0 at 256,
 // 53.4 / 46.0 at 637, 187 / 180 at 3072; FP32 22.7 / 14.0, 24.1 / 16.5, 30.5 /

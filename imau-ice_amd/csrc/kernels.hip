@@ -593,7 +593,7 @@ __global__ void __launch_bounds__(IMAU_WG) k_visc(const Member *__restrict__ mem
 // integrals are summed afterwards from LDS, in the same order with the same
 // rounding, so the results are the same bit for bit.  The column's 25 values
 // are loaded once per level, which costs nothing while the chip is idle.
-// 30 -> 8.4 us on 29x29 cells, 30 -> 15 on 401x41 (FP64, 15 levels).
+// 28 -> 8 us on 29x29 cells (4 tiles), 29 -> 13.5 on 401x41 (51; FP64, 15 levels).
 template <bool DIVA, bool THIRD, class T>
 __global__ void __launch_bounds__(IMAU_TJ *IMAU_LEVMAX) k_visc_lev(
     const Member *__restrict__ mem, const Tile *__restrict__ tiles, const KP kp, const Fields f,
@@ -1801,10 +1801,12 @@ template <class T>
 static void visc_tiles(const Launch &L, const Launch &LV, const KP &kp, const Fields &f, bool diva, const T *visc_in,
                        T *visc_out, const T *B3, const int *active) {
   const bool third = kp.n_flow == 3.0;
-  // few tiles: a wavefront per level instead of per column (the line's two sides stand at IMAU_LEVTILES)
-  if (kp.nz <= IMAU_LEVMAX && LV.ntiles <= IMAU_LEVTILES) {
+  // few tiles: a wavefront per level instead of per column, except where a column
+  // shares its power law (the lines' two sides stand at IMAU_LEVTILES)
+  const bool pays = diva || third || sizeof(T) == 4;
+  if (pays && kp.nz <= IMAU_LEVMAX && LV.ntiles <= IMAU_LEVTILES) {
     auto kl = diva ? (third ? k_visc_lev<true, true, T> : k_visc_lev<true, false, T>)
-                   : (third ? k_visc_lev<false, true, T> : k_visc_lev<false, false, T>);
+                   : (third ? k_visc_lev<false, true, T> : k_visc_lev<false, sizeof(T) == 8, T>);  // FP64 with n != 3: never taken
     hipLaunchKernelGGL(kl, dim3(LV.ntiles * IMAU_VTI), dim3(IMAU_TJ, kp.nz), 0, L.s, L.mem, LV.tiles, kp, f, visc_in,
                        visc_out, B3, active);
     return;

@@ -58,11 +58,11 @@ def test_every_tile_height_gives_the_same_solve(ctx, precision):
 @pytest.mark.parametrize("precision", ["fp64", "mixed_visc"])
 @pytest.mark.parametrize("shape,nz,dyn,n_flow", [((9, 12), 15, "DIVA", 3.0), ((9, 64), 16, "DIVA", 3.0),
                                                  ((17, 65), 2, "DIVA", 2.5), ((8, 129), 15, "SSA", 3.0),
-                                                 ((26, 40), 5, "SSA", 2.5)])
+                                                 ((26, 40), 5, "SSA", 2.5), ((255, 70), 15, "DIVA", 3.0)])
 def test_viscosity_by_level_equals_by_column(ctx, shape, nz, dyn, n_flow, precision):
     """A few tiles take one wavefront per level, many one lane per column: a
     small member solved alone and beside a large one (1, 2 and 3 tile columns,
-    the fewest and most levels) ends in the same state bit for bit."""
+    the fewest and most levels, the most tiles) ends in the same state bit for bit."""
     z = np.linspace(0.0, 1.0, nz) ** 0.8
     cfg = geometry.synthetic_config(choice_ice_dynamics=dyn, n_flow=n_flow, zeta=[float(a) for a in z])
     config.set_config(cfg, stop_rule=1, nonlinear_rtol=1e-12, DIVA_visc_it_nit=4, precision=precision)
