@@ -586,9 +586,9 @@ void wire(imau_problem *P) {
 bool uses_ssa_field(int dyn) { return dyn == IMAU_DYN_SSA || dyn == IMAU_DYN_SIA_SSA; }
 
 // buffers that only some configurations use (GCR directions, Anderson
-// slots, the FP32 viscosity), allocated before a solve's first kernel since
-// DBuf::alloc synchronises the device: at create for the create-time
+// slots, the FP32 viscosity): allocated at create for the create-time
 // configuration, and at the start of a solve whose configuration needs more
+// (an allocation inside the loop would stop the host between launches)
 void reserve_buffers(imau_ctx *c, imau_problem *P, const imau_cfg *cfg) {
   const long long na = P->na, n3 = na * (long long)P->nz;
   if (cfg->DIVA_choice_matrix_solver != IMAU_SOLVER_SOR && cfg->ksp_type == 1 && !P->gcr_dirs.p)
@@ -1295,9 +1295,9 @@ struct Solver {
     }
   }
 
-  // preconditioner application z = M^-1 y shared by the Krylov methods
-  // V-cycles captured as HIP graphs, one per (operands, precision, smoother
-  // form) seen in this solve: the kernel parameters, coefficients and levels
+  // GCR's preconditioner application z = M^-1 y (krylov_solve launches its
+  // V-cycles kernel by kernel).  V-cycles captured as HIP graphs, one per
+  // (operands, precision, smoother form) seen in this solve: the kernel parameters, coefficients and levels
   // are fixed for the solve, the activity flags are read from device memory
   // at replay.  Released with the solver.
   struct VGraph {

@@ -187,10 +187,11 @@ typedef struct imau_cfg {
   double  stall_drop;      /* > 1                                            */
   double  stall_relax;     /* DIVA_visc_it_relax of a restarted member's
                               unmixed Picard steps (0 = DIVA_visc_it_relax)  */
-  int32_t mg_graph;        /* 1: each multigrid V-cycle is replayed from a HIP
-                              graph captured on its first use in a solve (one
-                              launch instead of one per kernel); 0: launched
-                              kernel by kernel.  Identical results          */
+  int32_t mg_graph;        /* 1: each multigrid V-cycle of GCR (ksp_type 1) is
+                              replayed from a HIP graph captured on its first
+                              use in a solve (one launch instead of one per
+                              kernel); 0, and under BiCGStab: launched kernel
+                              by kernel.  Identical results                 */
 } imau_cfg;
 
 /* The fields of type_ice_model (src/data_types_module.f90:56-325) that the
@@ -288,9 +289,10 @@ const char *imau_vel_last_error(const imau_ctx *ctx);
  * processed (members that have converged are skipped), since the previous
  * call; then resets the counters and
  * selects what is timed next: IMAU_TIME_OFF, IMAU_TIME_SMOOTHER (one
- * fine-level smoother sweep: the five colour launches of a multigrid sweep,
- * a tile Gauss-Seidel application, or one SOR sweep) or IMAU_TIME_VISC (the
- * 3D viscosity kernel of a Picard iteration). */
+ * fine-level smoother sweep: the launch that also restricts its residual, the
+ * five colour launches of a multigrid sweep where mg_smoother is 1, a tile
+ * Gauss-Seidel application, or one SOR sweep) or IMAU_TIME_VISC (the 3D
+ * viscosity of a Picard iteration with its strain rates). */
 enum { IMAU_TIME_OFF = 0, IMAU_TIME_SMOOTHER = 1, IMAU_TIME_VISC = 2 };
 int  imau_vel_kernel_timing(imau_ctx *ctx, int32_t what, int64_t *launches, double *ms, int64_t *cells);
 
