@@ -86,6 +86,7 @@ class DevPool {
     }
     if (!p && hipMalloc(&p, cap) != hipSuccess) {
       (void)hipGetLastError();
+      Scarce scarce;  // no thread keeps a block until the second try is over
       trim_all();
       HIPCHK(hipMalloc(&p, cap));
     }
@@ -100,7 +101,7 @@ class DevPool {
   void put(void *p, size_t cap, bool keep) noexcept {
     if (keep) {
       std::lock_guard<std::mutex> lock(mu_);
-      if (open_ && cap <= limit_) try {
+      if (open_ && cap <= limit_ && open_pools().scarce == 0) try {
         kept_.push_back(Block{p, cap});
         total_ += cap;
         p = nullptr;
@@ -148,11 +149,16 @@ class DevPool {
   struct OpenPools {
     std::mutex mu;  // taken before a pool's own
     std::vector<DevPool *> all;
+    std::atomic<int> scarce{0};
   };
   static OpenPools &open_pools() {
     static OpenPools *p = new OpenPools;  // outlives every static object that may still hold a pool
     return *p;
   }
+  struct Scarce {
+    Scarce() { ++open_pools().scarce; }
+    ~Scarce() { --open_pools().scarce; }
+  };
   static void trim_all() {
     std::lock_guard<std::mutex> lock(open_pools().mu);
     for (DevPool *p : open_pools().all) p->trim(0);

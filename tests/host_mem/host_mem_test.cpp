@@ -233,7 +233,7 @@ int closed() {
 // allocations of several threads and contexts, with less memory than they want to keep
 int pool_threads() {
   const Pool pools[2] = {new_pool(), new_pool()};
-  fake::st().limit = 24 << 20;
+  fake::st().limit = 15 << 20;  // 4 x (1.25 x 2 + 1) MiB in use at most
   std::atomic<int> bad{0};
   std::vector<std::thread> ts;
   for (unsigned q = 0; q < 4; ++q)
